@@ -9,19 +9,19 @@
 //   scan            bucket offsets (hipCUB)
 //   k_coll_fill     bucket lists of particle indices
 //   k_coll_classify cells with both species into lists by size (at most 16,
-//                   64, 256 or more particles of either species; a cell
-//                   missing a species ends its r-row as the reference's
+//                   32, 64, 128, 256 or more particles of either species; a
+//                   cell missing a species ends its r-row as the reference's
 //                   `break` does)
-//   k_coll_prep     per listed cell (one lane per cell of at most 16, one
-//                   wavefront with an LDS stage per cell of at most 64 or
-//                   256, one workgroup with a global stage per larger cell):
-//                   shuffle each bucket by sorting on
+//   k_coll_prep     per group of listed cells (1024 particle slots of one
+//                   size class, one workgroup; a cell above 256 has a
+//                   workgroup and a global stage of its own):
+//                   shuffle each bucket by ranking its particles on
 //                   a Philox key of (particle id, pass), per-cell sums in the
 //                   shuffled order, density / temperature / Debye length, and
 //                   the first cell of each r-row whose values are not normal
 //                   (the reference's `break` ends the rest of that row)
-//   k_coll_pairs    per listed cell, grouped the same way: the reference's
-//                   pair schedule with lanes on independent pair chains,
+//   k_coll_pairs    per group, the same way: the reference's pair schedule as
+//                   dense lists of independent pairs over the group's cells,
 //                   velocities staged in FP64; pair q of global cell c draws
 //                   the uniforms Philox(seed; c << 24 | q, 2 pass + 1)
 #include <hip/hip_runtime.h>
@@ -169,56 +169,9 @@ __device__ __forceinline__ CellPos cell_pos(const Geom &g, long c) {
   return q;
 }
 
-// ascending bitonic sort of n (<= COLL_MAXC) keys with their indices, by
-// one wavefront
-__device__ void wave_sort(uint64_t *key, uint32_t *idx, int n) {
-  int P = 1;
-  while (P < n) P <<= 1;
-  for (int t = n + (int)threadIdx.x; t < P; t += COLL_BLOCK) {
-    key[t] = ~0ull;
-    idx[t] = 0xFFFFFFFFu;
-  }
-  __syncthreads();
-  for (int k = 2; k <= P; k <<= 1)
-    for (int j = k >> 1; j > 0; j >>= 1) {
-      for (int t = threadIdx.x; t < P; t += COLL_BLOCK) {
-        int l = t ^ j;
-        if (l > t) {
-          bool asc = (t & k) == 0;
-          uint64_t a = key[t], b = key[l];
-          // (key, index) order: padding (key ~0, index ~0) stays behind
-          // every real entry
-          bool gt = a > b || (a == b && idx[t] > idx[l]);
-          if (asc ? gt : !gt) {
-            key[t] = b; key[l] = a;
-            uint32_t x = idx[t]; idx[t] = idx[l]; idx[l] = x;
-          }
-        }
-      }
-      __syncthreads();
-    }
-}
-
 struct CellSums {
   double amount, energy, m[3];
 };
-
-// sequential sums in bucket order (collect_weighted_params_tot_grid)
-__device__ CellSums cell_sums(const double *vx, const double *vy, const double *vz, const double *w, int n,
-                              double mass) {
-  CellSums t{0, 0, {0, 0, 0}};
-  for (int k = 0; k < n; ++k) {
-    double vr = vx[k], vphi = vy[k], vzz = vz[k];
-    double v_sq = vr * vr + vphi * vphi + vzz * vzz;
-    double weighted_m = w[k] * mass;
-    t.m[0] += weighted_m * vr;
-    t.m[1] += weighted_m * vphi;
-    t.m[2] += weighted_m * vzz;
-    t.amount += w[k];
-    t.energy += weighted_m * v_sq / 2;
-  }
-  return t;
-}
 
 // per-cell values kept between the two kernels
 constexpr int TOT = 16;   // a_e E_e m_e[3] a_i E_i m_i[3] dens_e dens_i debye dens_e^(2/3) dens_i^(2/3)
@@ -231,12 +184,14 @@ struct CellStageT {
 };
 using CellStage = CellStageT<COLL_MAXC>;
 
-// cells are processed by size class: at most 16, 64 or COLL_MAXC particles
-// of either species (smaller stages leave room for more wavefronts per CU)
-constexpr int COLL_CLASSES = 4;
-// class 0: one lane per cell; 1, 2: a wavefront per cell, LDS stage; 3
-// (crowded): a workgroup per cell, stage in global memory
-constexpr int COLL_CLASS_MAXC[COLL_CLASSES] = {16, 64, COLL_MAXC, INT_MAX};
+// cells are processed by size class: at most 16, 32, 64, 128 or COLL_MAXC
+// particles of either species (a workgroup takes as many cells as fill its
+// stage), the last class (crowded) a workgroup per cell, staged in global
+// memory
+constexpr int COLL_CLASSES = 6;
+constexpr int COLL_GROUP_CLASSES = COLL_CLASSES - 1;
+constexpr int COLL_CLASS0_SHIFT = 4;   // class k < 5 holds cells of at most 16 << k particles
+static_assert((16 << (COLL_GROUP_CLASSES - 1)) == COLL_MAXC, "the last grouped class is COLL_MAXC");
 // particles of all crowded cells of one pass that the global stage holds;
 // beyond it a pass raises ERR_COLL_OVERFLOW
 constexpr long COLL_CROWD_CAP = 1L << 22;
@@ -254,24 +209,6 @@ __device__ __forceinline__ void stage_species(const V &v, const uint32_t *perm, 
     S.vx[s][k] = vv[0]; S.vy[s][k] = vv[1]; S.vz[s][k] = vv[2];
     S.w[s][k] = v.w(p);
   }
-}
-
-// shuffle of one bucket: order by (Philox key, low id bits)
-template <class V>
-__device__ __forceinline__ void shuffle_bucket(const V &v, uint32_t *perm, uint32_t o, int n, uint64_t seed,
-                                               uint64_t step, uint64_t *skey, uint32_t *sidx) {
-  for (int k = threadIdx.x; k < n; k += COLL_BLOCK) {
-    uint32_t p = perm[o + k];
-    uint64_t id = v.id(p);
-    uint32_t ph[4];
-    philox4x32(id, (uint32_t)(2 * step), seed, ph);
-    skey[k] = ((uint64_t)ph[0] << 32) | (id & 0xFFFFFFFFull);
-    sidx[k] = p;
-  }
-  __syncthreads();
-  wave_sort(skey, sidx, n);
-  for (int k = threadIdx.x; k < n; k += COLL_BLOCK) perm[o + k] = sidx[k];
-  __syncthreads();
 }
 
 // Cells with particles of both species go to the list of their size class;
@@ -296,7 +233,7 @@ __global__ void k_coll_classify(Geom g, const uint32_t *off_e, const uint32_t *o
       } else {
         const int m = max(ne, ni);
         cls = 0;
-        while (m > COLL_CLASS_MAXC[cls]) ++cls;
+        while (cls < COLL_GROUP_CLASSES && m > (16 << cls)) ++cls;
         if (cls == COLL_CLASSES - 1) {
           // a range of the crowded stage (counts[COLL_CLASSES] particles used)
           const uint32_t need = (uint32_t)(ne + ni);
@@ -347,172 +284,220 @@ __device__ __forceinline__ void cell_stats(const Geom &g, long c, const CellSums
   if (bad) atomicMin(&row_bad[(long)q.d * g.nr + q.i], q.j);
 }
 
-template <class V, int MAXC>
-__global__ void __launch_bounds__(COLL_BLOCK) k_coll_prep(Geom g, V ve, V vi, const uint32_t *off_e,
-                                                          const uint32_t *off_i, uint32_t *perm_e, uint32_t *perm_i,
-                                                          double m_e, double m_i, uint64_t seed, PassNo pass,
-                                                          double *tot, int *row_bad, const uint32_t *list,
-                                                          const uint32_t *count, StepState *st,
-                                                          const unsigned long long *gate) {
-  const uint64_t step = pass.get();
-  __shared__ uint64_t skey[MAXC];
-  __shared__ CellStageT<MAXC> S;
-  if (gate_closed(gate)) return;
-  const uint32_t nlist = *count;
-  for (uint32_t li = blockIdx.x; li < nlist; li += gridDim.x) {
-    const long c = list[li];
-    int nn[2] = {(int)(off_e[c + 1] - off_e[c]), (int)(off_i[c + 1] - off_i[c])};
-    shuffle_bucket(ve, perm_e, off_e[c], nn[0], seed, step, skey, S.idx[0]);
-    shuffle_bucket(vi, perm_i, off_i[c], nn[1], seed, step, skey, S.idx[1]);
-    stage_species(ve, perm_e, off_e[c], nn[0], 0, S);
-    stage_species(vi, perm_i, off_i[c], nn[1], 1, S);
-    __syncthreads();
-    if (threadIdx.x == 0) {
-      CellSums te = cell_sums(S.vx[0], S.vy[0], S.vz[0], S.w[0], nn[0], m_e);
-      CellSums ti = cell_sums(S.vx[1], S.vy[1], S.vz[1], S.w[1], nn[1], m_i);
-      double sum_el = 0, sum_ion = 0;
-      for (int k = 0; k < nn[0]; ++k) sum_el += S.w[0][k];
-      for (int k = 0; k < nn[1]; ++k) sum_ion += S.w[1][k];
-      cell_stats(g, c, te, ti, sum_el, sum_ion, tot, row_bad);
+// ---------------------------------------------------------------------------
+// Grouped cells: a workgroup takes as many cells of one size class as fit its
+// stage (512 or 1024 particle slots) at their class's size -- of 1024, 32 cells
+// of at most 16 particles per species, ... 2 cells of at most 256.  Entry 2 g + s is species
+// s of the group's cell g; its particles take the slots start[e] .. + n[e],
+// one entry after another (starts at multiples of 4).
+// ---------------------------------------------------------------------------
+constexpr int COLL_GROUP_BLOCK = 256;
+static_assert(COLL_GROUP_BLOCK == 4 * 64, "a wavefront per stage list");
+constexpr int COLL_GROUP_SLOTS = 1024;   // k_coll_pairs
+constexpr int COLL_PREP_SLOTS = 512;     // k_coll_prep
+constexpr int COLL_GROUP_CELLS = COLL_GROUP_SLOTS >> (COLL_CLASS0_SHIFT + 1);   // the most cells of a group
+static_assert(COLL_GROUP_CELLS * 2 <= 64, "a group's (cell, species) entries fit a wavefront");
+
+// group number `it` over the class lists: its cells and their list entries
+// (false: past the last group)
+struct CellGroup {
+  int cells;
+  const uint32_t *list;
+};
+template <int SLOTS>
+__device__ __forceinline__ bool cell_group(uint32_t it, const uint32_t *lists, const uint32_t *counts, long ncells,
+                                           CellGroup &G) {
+  // the largest cells first: their groups run longest
+  for (int cls = COLL_GROUP_CLASSES - 1; cls >= 0; --cls) {
+    const uint32_t n = counts[cls];
+    const uint32_t per = SLOTS >> (COLL_CLASS0_SHIFT + cls + 1);
+    const uint32_t ng = (n + per - 1) / per;
+    if (it < ng) {
+      G.cells = (int)min(per, n - it * per);
+      G.list = lists + (long)cls * ncells + it * per;
+      return true;
     }
-    __syncthreads();
+    it -= ng;
   }
+  return false;
 }
 
-// ---------------------------------------------------------------------------
-// Tiny cells (at most COLL_TINY particles of either species, e.g. the sparse
-// rows near the axis of a plasma uniform in r^2): one lane per cell, so a
-// wavefront works on 64 cells.  The shuffle sorts the keys in registers
-// (odd-even transposition network, fully unrolled); the pairs run the same
-// schedule as the wavefront kernels, one pair after another, on velocities
-// staged in FP64 in a global per-lane array laid out [slot][lane] (adjacent
-// lanes, adjacent addresses).  Pairs of one schedule phase touch disjoint
-// particles and draw by ordinal, so the results equal the wavefront path's.
-// ---------------------------------------------------------------------------
-constexpr int COLL_TINY = 16;
-constexpr int COLL_LANE_BLOCK = 256;
-constexpr int COLL_LANE_SLOTS = 4 * 2 * COLL_TINY;   // vx, vy, vz, w of both species
-static_assert(COLL_CLASS_MAXC[0] == COLL_TINY, "class 0 is the lane-per-cell class");
-
-template <class V>
-__device__ __forceinline__ void lane_shuffle(const V &v, uint32_t *perm, uint32_t o, int n, uint64_t seed,
-                                             uint64_t step, uint32_t idx[COLL_TINY]) {
-  uint64_t key[COLL_TINY];
-#pragma unroll
-  for (int k = 0; k < COLL_TINY; ++k) {
-    key[k] = ~0ull;
-    idx[k] = 0xFFFFFFFFu;
-    if (k < n) {
-      const uint32_t p = perm[o + k];
-      const uint64_t id = v.id(p);
-      uint32_t ph[4];
-      philox4x32(id, (uint32_t)(2 * step), seed, ph);
-      key[k] = ((uint64_t)ph[0] << 32) | (id & 0xFFFFFFFFull);
-      idx[k] = p;
-    }
+// exclusive sum over a wavefront of one value per lane into out[0 .. 64]
+__device__ __forceinline__ void wave_starts(int v, int lane, int out[65]) {
+  int x = v;
+  for (int d = 1; d < 64; d <<= 1) {
+    const int y = __shfl_up(x, d, 64);
+    if (lane >= d) x += y;
   }
-  // (key, index) ascending, padding last: the order wave_sort gives
-#pragma unroll
-  for (int r = 0; r < COLL_TINY; ++r)
-#pragma unroll
-    for (int k = r & 1; k + 1 < COLL_TINY; k += 2) {
-      const bool gt = key[k] > key[k + 1] || (key[k] == key[k + 1] && idx[k] > idx[k + 1]);
-      if (gt) {
-        const uint64_t tk = key[k]; key[k] = key[k + 1]; key[k + 1] = tk;
-        const uint32_t ti = idx[k]; idx[k] = idx[k + 1]; idx[k + 1] = ti;
+  out[lane + 1] = x;
+  if (lane == 0) out[0] = 0;
+}
+// the e with start[e] <= t < start[e + 1]
+__device__ __forceinline__ int entry_of(const int start[65], int t) {
+  int e = 0, hi = 64;
+  while (hi - e > 1) {
+    const int mid = (e + hi) >> 1;
+    if (start[mid] <= t) e = mid;
+    else hi = mid;
+  }
+  return e;
+}
+
+// the buckets of a group: offset into perm, particles, first slot
+struct GroupEntries {
+  uint32_t off[64];
+  int n[64];
+  int start[65];
+  // by the first wavefront; a barrier follows
+  __device__ __forceinline__ void load(const CellGroup &G, const uint32_t *off_e, const uint32_t *off_i) {
+    if (threadIdx.x >= 64) return;
+    const int e = threadIdx.x;
+    int cnt = 0;
+    if (e < 2 * G.cells) {
+      const long c = G.list[e >> 1];
+      const uint32_t *o = (e & 1) ? off_i : off_e;
+      off[e] = o[c];
+      cnt = (int)(o[c + 1] - o[c]);
+    }
+    n[e] = cnt;
+    wave_starts((cnt + 3) & ~3, e, start);
+  }
+};
+
+// Shuffle and cell sums.  A particle's place is its rank among its bucket's
+// 32-bit Philox keys (n comparisons against broadcast LDS reads of four keys,
+// no barrier in the loop; equal keys, found by two particles claiming one
+// place, are ranked again by (key, id, index)).  The sums run in the shuffled
+// order, one thread per (quantity, species, cell).  Bound by latency: the
+// bitonic sort and one-thread sums of a wavefront per cell took 6.2 ms per pass
+// on a million cells of 32 + 32 FP64 particles on average (16 wavefronts per CU
+// at a 1024-slot stage still 2.7), this 2.1 with k_coll_stats.
+template <class V>
+__global__ void __launch_bounds__(COLL_GROUP_BLOCK) k_coll_prep(Geom g, V ve, V vi, const uint32_t *off_e,
+                                                                const uint32_t *off_i, uint32_t *perm_e,
+                                                                uint32_t *perm_i, double m_e, double m_i,
+                                                                uint64_t seed, PassNo pass, double *tot,
+                                                                const uint32_t *lists, const uint32_t *counts,
+                                                                long ncells, const unsigned long long *gate) {
+  __shared__ GroupEntries E;
+  __shared__ __align__(16) uint32_t skey[COLL_PREP_SLOTS];
+  __shared__ uint32_t sidx[COLL_PREP_SLOTS], claim[COLL_PREP_SLOTS];
+  __shared__ double sx[COLL_PREP_SLOTS], sy[COLL_PREP_SLOTS], sz[COLL_PREP_SLOTS], sw[COLL_PREP_SLOTS];
+  __shared__ int tie;
+  if (gate_closed(gate)) return;
+  const uint64_t step = pass.get();
+  CellGroup G;
+  for (uint32_t it = blockIdx.x; cell_group<COLL_PREP_SLOTS>(it, lists, counts, ncells, G); it += gridDim.x) {
+    const int entries = 2 * G.cells;
+    E.load(G, off_e, off_i);
+    if (threadIdx.x == 0) tie = 0;
+    __syncthreads();
+    const int slots = E.start[64];
+    for (int t = threadIdx.x; t < slots; t += COLL_GROUP_BLOCK) {
+      const int e = entry_of(E.start, t), k = t - E.start[e];
+      uint32_t key = 0xFFFFFFFFu;
+      claim[t] = 0;
+      if (k < E.n[e]) {
+        const uint32_t p = ((e & 1) ? perm_i : perm_e)[E.off[e] + k];
+        const uint64_t id = (e & 1) ? vi.id(p) : ve.id(p);
+        uint32_t ph[4];
+        philox4x32(id, (uint32_t)(2 * step), seed, ph);
+        key = ph[0];
+        sidx[t] = p;
       }
+      skey[t] = key;
     }
-#pragma unroll
-  for (int k = 0; k < COLL_TINY; ++k)
-    if (k < n) perm[o + k] = idx[k];
-}
-
-// cell_sums of the shuffled particles, and their weight sum
-template <class V>
-__device__ __forceinline__ CellSums lane_sums(const V &v, const uint32_t idx[COLL_TINY], int n, double mass,
-                                              double &sum_w) {
-  CellSums t{0, 0, {0, 0, 0}};
-  sum_w = 0;
-#pragma unroll
-  for (int k = 0; k < COLL_TINY; ++k) {
-    if (k >= n) break;
-    double vv[3];
-    v.load(idx[k], vv);
-    const double w = v.w(idx[k]);
-    double vr = vv[0], vphi = vv[1], vzz = vv[2];
-    double v_sq = vr * vr + vphi * vphi + vzz * vzz;
-    double weighted_m = w * mass;
-    t.m[0] += weighted_m * vr;
-    t.m[1] += weighted_m * vphi;
-    t.m[2] += weighted_m * vzz;
-    t.amount += w;
-    t.energy += weighted_m * v_sq / 2;
-    sum_w += w;
+    __syncthreads();
+    for (int t = threadIdx.x; t < slots; t += COLL_GROUP_BLOCK) {
+      const int e = entry_of(E.start, t), base = E.start[e], n = E.n[e];
+      if (t - base >= n) continue;
+      const uint32_t key = skey[t], p = sidx[t];
+      double v3[3], w;
+      if (e & 1) { vi.load(p, v3); w = vi.w(p); }
+      else { ve.load(p, v3); w = ve.w(p); }
+      int r = 0;
+#pragma unroll 4
+      for (int j = 0; j < n; j += 4) {
+        const uint4 q = *(const uint4 *)(skey + base + j);
+        r += (int)(q.x < key) + (int)(q.y < key) + (int)(q.z < key) + (int)(q.w < key);
+      }
+      if (atomicExch(&claim[base + r], 1u)) tie = 1;
+      ((e & 1) ? perm_i : perm_e)[E.off[e] + r] = p;
+      sx[base + r] = v3[0]; sy[base + r] = v3[1]; sz[base + r] = v3[2];
+      sw[base + r] = w;
+    }
+    __syncthreads();
+    if (tie) {
+      // two particles of a bucket drew the same key: rank by (key, low id bits, index)
+      for (int t = threadIdx.x; t < slots; t += COLL_GROUP_BLOCK) {
+        const int e = entry_of(E.start, t), base = E.start[e], n = E.n[e];
+        if (t - base >= n) continue;
+        const uint32_t key = skey[t], p = sidx[t];
+        const uint32_t id = (uint32_t)((e & 1) ? vi.id(p) : ve.id(p));
+        int r = 0;
+        for (int j = 0; j < n; ++j) {
+          bool less = skey[base + j] < key;
+          if (skey[base + j] == key && base + j != t) {
+            const uint32_t pj = sidx[base + j], idj = (uint32_t)((e & 1) ? vi.id(pj) : ve.id(pj));
+            less = idj < id || (idj == id && pj < p);
+          }
+          r += less ? 1 : 0;
+        }
+        double v3[3], w;
+        if (e & 1) { vi.load(p, v3); w = vi.w(p); }
+        else { ve.load(p, v3); w = ve.w(p); }
+        ((e & 1) ? perm_i : perm_e)[E.off[e] + r] = p;
+        sx[base + r] = v3[0]; sy[base + r] = v3[1]; sz[base + r] = v3[2];
+        sw[base + r] = w;
+      }
+      __syncthreads();
+    }
+    // collect_weighted_params_tot_grid: 0 weight, 1 energy, 2-4 momentum
+    for (int t = threadIdx.x; t < 5 * 64; t += COLL_GROUP_BLOCK) {
+      const int q = t >> 6, e = t & 63;
+      if (e >= entries) continue;
+      const int n = E.n[e], base = E.start[e];
+      const double mass = (e & 1) ? m_i : m_e;
+      const double *v = q == 2 ? sx : q == 3 ? sy : sz;
+      double a = 0;
+      if (q >= 2) {
+#pragma unroll 4
+        for (int k = 0; k < n; ++k) a += sw[base + k] * mass * v[base + k];
+      } else if (q == 0) {
+#pragma unroll 4
+        for (int k = 0; k < n; ++k) a += sw[base + k];
+      } else {
+#pragma unroll 4
+        for (int k = 0; k < n; ++k) {
+          const double vr = sx[base + k], vphi = sy[base + k], vz = sz[base + k];
+          const double v_sq = vr * vr + vphi * vphi + vz * vz;
+          a += sw[base + k] * mass * v_sq / 2;
+        }
+      }
+      tot[(long)G.list[e >> 1] * TOT + 5 * (e & 1) + q] = a;
+    }
+    __syncthreads();
   }
-  return t;
 }
 
-template <class V>
-__global__ void __launch_bounds__(COLL_LANE_BLOCK) k_coll_prep_lane(Geom g, V ve, V vi, const uint32_t *off_e,
-                                                                    const uint32_t *off_i, uint32_t *perm_e,
-                                                                    uint32_t *perm_i, double m_e, double m_i,
-                                                                    uint64_t seed, PassNo pass, double *tot,
-                                                                    int *row_bad, const uint32_t *list,
-                                                                    const uint32_t *count,
-                                                                    const unsigned long long *gate) {
-  const uint64_t step = pass.get();
+// density, temperature and Debye length of the grouped classes' cells from
+// k_coll_prep's sums, a lane per cell (in k_coll_prep the few cells of a group
+// kept 4 lanes of a wavefront busy for it)
+__global__ void __launch_bounds__(256) k_coll_stats(Geom g, double *tot, int *row_bad, const uint32_t *lists,
+                                                    const uint32_t *counts, long ncells,
+                                                    const unsigned long long *gate) {
   if (gate_closed(gate)) return;
-  const uint32_t nlist = *count;
-  for (uint32_t li = blockIdx.x * blockDim.x + threadIdx.x; li < nlist; li += gridDim.x * blockDim.x) {
-    const long c = list[li];
-    const int ne = (int)(off_e[c + 1] - off_e[c]), ni = (int)(off_i[c + 1] - off_i[c]);
-    uint32_t ie[COLL_TINY], ii[COLL_TINY];
-    lane_shuffle(ve, perm_e, off_e[c], ne, seed, step, ie);
-    lane_shuffle(vi, perm_i, off_i[c], ni, seed, step, ii);
-    double sum_el, sum_ion;
-    const CellSums te = lane_sums(ve, ie, ne, m_e, sum_el);
-    const CellSums ti = lane_sums(vi, ii, ni, m_i, sum_ion);
-    cell_stats(g, c, te, ti, sum_el, sum_ion, tot, row_bad);
+  for (int cls = 0; cls < COLL_GROUP_CLASSES; ++cls) {
+    const uint32_t n = counts[cls];
+    for (uint32_t t = blockIdx.x * blockDim.x + threadIdx.x; t < n; t += gridDim.x * blockDim.x) {
+      const long c = lists[(long)cls * ncells + t];
+      const double *s = tot + c * TOT;
+      const CellSums te{s[0], s[1], {s[2], s[3], s[4]}}, ti{s[5], s[6], {s[7], s[8], s[9]}};
+      cell_stats(g, c, te, ti, te.amount, ti.amount, tot, row_bad);
+    }
   }
 }
 
-// who runs a cell's loops: a wavefront (lanes split the independent pairs
-// of a phase) or a single lane (everything in order)
-template <int N>
-struct GroupTeam {
-  static constexpr int step = N;
-  __device__ __forceinline__ int first() const { return (int)threadIdx.x; }
-  __device__ __forceinline__ void sync() const { __syncthreads(); }
-};
-using WaveTeam = GroupTeam<COLL_BLOCK>;
-using BlockTeam = GroupTeam<COLL_CROWD_BLOCK>;
-struct LaneTeam {
-  static constexpr int step = 1;
-  __device__ __forceinline__ int first() const { return 0; }
-  __device__ __forceinline__ void sync() const {}
-};
-
-// a cell's staged FP64 particles: the wavefront's LDS stage, or a lane's
-// slots of the global array
-template <int MAXC>
-struct WaveStage {
-  CellStageT<MAXC> *S;
-  __device__ __forceinline__ double &vx(int s, int k) const { return S->vx[s][k]; }
-  __device__ __forceinline__ double &vy(int s, int k) const { return S->vy[s][k]; }
-  __device__ __forceinline__ double &vz(int s, int k) const { return S->vz[s][k]; }
-  __device__ __forceinline__ double &w(int s, int k) const { return S->w[s][k]; }
-};
-struct LaneStage {
-  double *b;     // this lane's slot 0
-  long stride;   // lanes of the launch
-  __device__ __forceinline__ double &at(int c, int s, int k) const {
-    return b[(long)((c * 2 + s) * COLL_TINY + k) * stride];
-  }
-  __device__ __forceinline__ double &vx(int s, int k) const { return at(0, s, k); }
-  __device__ __forceinline__ double &vy(int s, int k) const { return at(1, s, k); }
-  __device__ __forceinline__ double &vz(int s, int k) const { return at(2, s, k); }
-  __device__ __forceinline__ double &w(int s, int k) const { return at(3, s, k); }
-};
 struct CrowdStage {
   double *b;     // the cell's range of the crowded stage
   int n0;        // electrons first, then ions
@@ -521,6 +506,19 @@ struct CrowdStage {
   __device__ __forceinline__ double &vy(int s, int k) const { return at(1, s, k); }
   __device__ __forceinline__ double &vz(int s, int k) const { return at(2, s, k); }
   __device__ __forceinline__ double &w(int s, int k) const { return at(3, s, k); }
+};
+
+__device__ __forceinline__ uint32_t like_pairs(int n) {
+  if (n % 2 == 0) return (uint32_t)(n / 2);
+  return (uint32_t)((n >= 3 ? 3 : 0) + (n >= 5 ? (n - 3) / 2 : 0));
+}
+
+// the threads that run a crowded cell's loops split the independent pairs of
+// a phase
+struct BlockTeam {
+  static constexpr int step = COLL_CROWD_BLOCK;
+  __device__ __forceinline__ int first() const { return (int)threadIdx.x; }
+  __device__ __forceinline__ void sync() const { __syncthreads(); }
 };
 
 // the pair schedule of one cell (collisionsP12.cpp:356-528)
@@ -532,8 +530,9 @@ struct PairRunner {
   double dens[2], debye, dt;
   uint64_t seed, step, gcell;
   int *err;
-  double dens23[2];   // n^(2/3) of electrons and ions
-  __device__ __forceinline__ void pair(int sa, int ka, int sb, int kb, uint32_t ord) {
+  P12Cell K[3];   // P12: electron, unlike, ion pairs
+  // out of line: the schedule calls it from several places
+  __device__ __noinline__ void pair(int sa, int ka, int sb, int kb, uint32_t ord) {
     PairDraws R;
     uint64_t ctr = (gcell << 24) | (uint64_t)(ord & 0xFFFFFFu);
     uint32_t draw = (uint32_t)(2 * step + 1);
@@ -543,7 +542,7 @@ struct PairRunner {
     double va[3] = {S.vx(sa, ka), S.vy(sa, ka), S.vz(sa, ka)};
     double vb[3] = {S.vx(sb, kb), S.vy(sb, kb), S.vz(sb, kb)};
     collide_pair<SCHEME>(m[sa], m[sb], q[sa], q[sb], va, S.w(sa, ka), vb, S.w(sb, kb), dens[sa], dens[sb],
-                         dens23[sa], dens23[sb], debye, dt, R, err);
+                         K[sa + sb], debye, dt, R, err);
     S.vx(sa, ka) = va[0]; S.vy(sa, ka) = va[1]; S.vz(sa, ka) = va[2];
     S.vx(sb, kb) = vb[0]; S.vy(sb, kb) = vb[1]; S.vz(sb, kb) = vb[2];
   }
@@ -563,11 +562,6 @@ struct PairRunner {
     }
   }
 };
-
-__device__ __forceinline__ uint32_t like_pairs(int n) {
-  if (n % 2 == 0) return (uint32_t)(n / 2);
-  return (uint32_t)((n >= 3 ? 3 : 0) + (n >= 5 ? (n - 3) / 2 : 0));
-}
 
 __device__ __forceinline__ int grp(unsigned f, float div) { return (int)floorf((float)f / div); }
 
@@ -684,15 +678,10 @@ __device__ CorrParams correct_params(const Stage &S, int s, int n, double mass, 
 
 template <class Stage, class Team>
 __device__ void correct_species(const Stage &S, const Team &T, int s, int n, double mass, const double *t) {
-  CorrParams P;
-  if constexpr (Team::step == 1) {
-    P = correct_params(S, s, n, mass, t);
-  } else {
-    __shared__ CorrParams shared_p;
-    if (threadIdx.x == 0) shared_p = correct_params(S, s, n, mass, t);
-    __syncthreads();
-    P = shared_p;
-  }
+  __shared__ CorrParams shared_p;
+  if (threadIdx.x == 0) shared_p = correct_params(S, s, n, mass, t);
+  __syncthreads();
+  const CorrParams P = shared_p;
   if (P.ok != 0.0) {
     const double alpha = P.alpha;
     for (int k = T.first(); k < n; k += Team::step) {
@@ -705,108 +694,253 @@ __device__ void correct_species(const Stage &S, const Team &T, int s, int n, dou
   T.sync();
 }
 
-template <int SCHEME, class V, int MAXC>
-__global__ void __launch_bounds__(COLL_BLOCK) k_coll_pairs(Geom g, V ve, V vi, const uint32_t *off_e,
-                                                           const uint32_t *off_i, const uint32_t *perm_e,
-                                                           const uint32_t *perm_i, double m_e, double m_i,
-                                                           double q_e, double q_i, uint64_t seed, PassNo pass,
-                                                           const double *tot, const int *row_bad,
-                                                           const uint32_t *list, const uint32_t *count,
-                                                           StepState *st, const unsigned long long *gate) {
-  const uint64_t step = pass.get();
-  __shared__ CellStageT<MAXC> S;
-  if (gate_closed(gate)) return;
-  const uint32_t nlist = *count;
-  int err = 0;
-  const WaveStage<MAXC> WS{&S};
-  const WaveTeam T;
-  for (uint32_t li = blockIdx.x; li < nlist; li += gridDim.x) {
-    const long c = list[li];
-    int nn[2] = {(int)(off_e[c + 1] - off_e[c]), (int)(off_i[c + 1] - off_i[c])};
-    stage_species(ve, perm_e, off_e[c], nn[0], 0, S);
-    stage_species(vi, perm_i, off_i[c], nn[1], 1, S);
-    __syncthreads();
-    const CellPos q = cell_pos(g, c);
-    const double *t = tot + c * TOT;
-    const bool active = q.j < row_bad[(long)q.d * g.nr + q.i];
-    if (active) {
-      PairRunner<SCHEME, WaveStage<MAXC>, WaveTeam> P{WS, T, {m_e, m_i}, {q_e, q_i}, {t[10], t[11]}, t[12], g.dt,
-                                                      seed, step, (uint64_t)q.cr * (uint64_t)g.Nz + (uint64_t)q.cz,
-                                                      &err, {t[13], t[14]}};
-      cell_pairs(P, nn[0], nn[1]);
+// The unlike pairs of a cell with N particles of the more numerous species
+// and n of the other (cases 2a / 2b): each of the n meets a chain of the N,
+// first particles of the reference's 1st group (c + 1 each), then of the 2nd
+// (c each).  No particle of the N is in two chains, so the chains are
+// independent and each runs in the reference's order.
+struct UnlikeChains {
+  int n, big, c;                 // chains, N, floor(N / n)
+  int big1, small1, big2;        // 1st group: particles of the N, of the n; 2nd group: of the N
+  __device__ __forceinline__ void set(int nel, int nion) {
+    const int lo = min(nel, nion), hi = max(nel, nion);
+    n = lo;
+    big = hi;
+    if (lo == hi || lo == 0) {
+      c = 1;
+      big1 = small1 = 0;
+      big2 = lo;
+      return;
     }
-    if (SCHEME == COLL_TA77S) {
-      // correct_velocities runs over every cell, ions first
-      correct_species(WS, T, 1, nn[1], m_i, t + 5);
-      correct_species(WS, T, 0, nn[0], m_e, t + 0);
-    }
-    for (int k = threadIdx.x; k < nn[0]; k += COLL_BLOCK) {
-      double v3[3] = {S.vx[0][k], S.vy[0][k], S.vz[0][k]};
-      ve.store(S.idx[0][k], v3);
-    }
-    for (int k = threadIdx.x; k < nn[1]; k += COLL_BLOCK) {
-      double v3[3] = {S.vx[1][k], S.vy[1][k], S.vz[1][k]};
-      vi.store(S.idx[1][k], v3);
-    }
-    __syncthreads();
+    const float ratio = (float)hi / (float)lo;
+    const double ci = (double)floorf(ratio);
+    const double cr = (double)ratio - ci;
+    c = (int)ci;
+    big1 = min((int)((ci + 1) * cr * lo), hi);
+    small1 = (int)(cr * lo);
+    big2 = min((int)(ci * (1 - cr) * lo), hi - big1);
   }
-  if (err && threadIdx.x == 0) atomicOr(&st->err, err);
-}
+  // chain e: pairs of the 1st and of both groups
+  __device__ __forceinline__ int first(int e) const { return min(max(big1 - e * (c + 1), 0), c + 1); }
+  __device__ __forceinline__ int length(int e) const {
+    return first(e) + (e >= small1 ? min(max(big2 - (e - small1) * c, 0), c) : 0);
+  }
+  // the N's particle (and pair ordinal) of pair j of chain e
+  __device__ __forceinline__ int partner(int e, int j) const {
+    const int f = first(e);
+    return j < f ? e * (c + 1) + j : big1 + (e - small1) * c + (j - f);
+  }
+  // chains that can hold more than one pair: every one for c > 1, else the 1st group's
+  __device__ __forceinline__ int long_chains() const { return c > 1 ? n : min(n, small1 + 1); }
+};
 
-// the pairs of tiny cells, one lane per cell; `stage` holds
-// COLL_LANE_SLOTS doubles per lane of the launch
+// what a pair takes from its cell
+struct CellStatsLds {
+  double dens[2], debye;
+  uint64_t gcell;
+  UnlikeChains chains;
+  int active;
+};
+
+// one bucket's slots, for correct_params
+struct SlotStage {
+  const double *x, *y, *z, *wt;
+  __device__ __forceinline__ double vx(int, int k) const { return x[k]; }
+  __device__ __forceinline__ double vy(int, int k) const { return y[k]; }
+  __device__ __forceinline__ double vz(int, int k) const { return z[k]; }
+  __device__ __forceinline__ double w(int, int k) const { return wt[k]; }
+};
+
+struct PairStage {
+  double vx[COLL_GROUP_SLOTS], vy[COLL_GROUP_SLOTS], vz[COLL_GROUP_SLOTS], w[COLL_GROUP_SLOTS];
+};
+
+// The pairs of a group run as stages of independent pairs or chains, each a
+// dense list over the group's cells that the workgroup's wavefronts take 64
+// entries at a time: the like pairs with the first of an odd bucket's three
+// chained ones, the rest of those chains, the first pair of every unlike
+// chain, the rest of the unlike chains.  Bound by FP64 instruction issue, so
+// what counts is how many of a wavefront's lanes hold a pair: a wavefront per
+// cell ran 40 + 40 particles as passes of 20, 20 and 40 of 64 lanes, and a lane
+// per cell the cells of up to 16.  One P12 pass over a million cells of 32 + 32
+// FP64 particles on average: 21.5 ms that way, 10.6 with the dense lists (and
+// the same pair arithmetic), 6.7 with p12_collide's shared reciprocals, 5.4 at
+// three wavefronts per SIMD (two without the limit; with the machine LICM pass
+// off, which kept the pair's FP64 constants in registers over the whole loop,
+// the limit spills 10 registers instead of 92; four spill 51 and measure the
+// same).
 template <int SCHEME, class V>
-__global__ void __launch_bounds__(COLL_LANE_BLOCK) k_coll_pairs_lane(
+__global__ void __launch_bounds__(COLL_GROUP_BLOCK) __attribute__((amdgpu_waves_per_eu(3))) k_coll_pairs(
     Geom g, V ve, V vi, const uint32_t *off_e, const uint32_t *off_i, const uint32_t *perm_e, const uint32_t *perm_i,
-    double m_e, double m_i, double q_e, double q_i, uint64_t seed, PassNo pass, const double *tot,
-    const int *row_bad, const uint32_t *list, const uint32_t *count, double *stage, StepState *st,
-    const unsigned long long *gate) {
-  const uint64_t step = pass.get();
+    double m_e, double m_i, double q_e, double q_i, uint64_t seed, PassNo pass, const double *tot, const int *row_bad,
+    const uint32_t *lists, const uint32_t *counts, long ncells, StepState *st, const unsigned long long *gate) {
+  constexpr int STAGES = 4;
+  __shared__ PairStage S;
+  __shared__ GroupEntries E;
+  __shared__ CellStatsLds C[COLL_GROUP_CELLS];
+  __shared__ P12Cell K[SCHEME == COLL_P12 ? COLL_GROUP_CELLS : 1][3];
+  __shared__ int pre[STAGES][65];
+  __shared__ uint32_t ticket[STAGES];
   if (gate_closed(gate)) return;
-  const uint32_t nlist = *count;
-  const long lanes = (long)gridDim.x * blockDim.x;
-  const long lane = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  const LaneStage S{stage + lane, lanes};
-  const LaneTeam T;
+  const uint64_t step = pass.get();
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   int err = 0;
-  for (long li = lane; li < (long)nlist; li += lanes) {
-    const long c = list[li];
-    const int nn[2] = {(int)(off_e[c + 1] - off_e[c]), (int)(off_i[c + 1] - off_i[c])};
-    const uint32_t o[2] = {off_e[c], off_i[c]};
-    for (int k = 0; k < nn[0]; ++k) {
-      const uint32_t p = perm_e[o[0] + k];
-      double vv[3];
-      ve.load(p, vv);
-      S.vx(0, k) = vv[0]; S.vy(0, k) = vv[1]; S.vz(0, k) = vv[2];
-      S.w(0, k) = ve.w(p);
+  CellGroup G;
+  for (uint32_t it = blockIdx.x; cell_group<COLL_GROUP_SLOTS>(it, lists, counts, ncells, G); it += gridDim.x) {
+    const int entries = 2 * G.cells;
+    E.load(G, off_e, off_i);
+    if (wave == 1 && lane < G.cells) {
+      const long c = G.list[lane];
+      const CellPos q = cell_pos(g, c);
+      const double *t = tot + c * TOT;
+      CellStatsLds &L = C[lane];
+      L.dens[0] = t[10]; L.dens[1] = t[11]; L.debye = t[12];
+      L.gcell = (uint64_t)q.cr * (uint64_t)g.Nz + (uint64_t)q.cz;
+      L.active = q.j < row_bad[(long)q.d * g.nr + q.i];
+      L.chains.set((int)(off_e[c + 1] - off_e[c]), (int)(off_i[c + 1] - off_i[c]));
     }
-    for (int k = 0; k < nn[1]; ++k) {
-      const uint32_t p = perm_i[o[1] + k];
-      double vv[3];
-      vi.load(p, vv);
-      S.vx(1, k) = vv[0]; S.vy(1, k) = vv[1]; S.vz(1, k) = vv[2];
-      S.w(1, k) = vi.w(p);
+    if (SCHEME == COLL_P12 && wave >= 2) {
+      const int t = (int)threadIdx.x - 128;
+      if (t < 3 * G.cells) {
+        const int i = t / 3, k = t - 3 * i;
+        K[i][k].set_species(k, m_e, m_i, q_e, q_i, tot + (long)G.list[i] * TOT + 10, g.dt);
+      }
     }
-    const CellPos q = cell_pos(g, c);
-    const double *t = tot + c * TOT;
-    if (q.j < row_bad[(long)q.d * g.nr + q.i]) {
-      PairRunner<SCHEME, LaneStage, LaneTeam> P{S, T, {m_e, m_i}, {q_e, q_i}, {t[10], t[11]}, t[12], g.dt,
-                                                seed, step, (uint64_t)q.cr * (uint64_t)g.Nz + (uint64_t)q.cz, &err,
-                                                {t[13], t[14]}};
-      cell_pairs(P, nn[0], nn[1]);
+    if (threadIdx.x < STAGES) ticket[threadIdx.x] = 0;
+    __syncthreads();
+    const int slots = E.start[64];
+    for (int t = threadIdx.x; t < slots; t += COLL_GROUP_BLOCK) {
+      const int e = entry_of(E.start, t), k = t - E.start[e];
+      if (k >= E.n[e]) continue;
+      const uint32_t p = ((e & 1) ? perm_i : perm_e)[E.off[e] + k];
+      double v3[3], w;
+      if (e & 1) { vi.load(p, v3); w = vi.w(p); }
+      else { ve.load(p, v3); w = ve.w(p); }
+      S.vx[t] = v3[0]; S.vy[t] = v3[1]; S.vz[t] = v3[2];
+      S.w[t] = w;
+    }
+    // list starts of the stages, a wavefront each: (cell, species) entries of
+    // stages 0 and 1, cells of 2 and 3
+    {
+      int v = 0;
+      if (wave < 2) {
+        if (lane < entries && C[lane >> 1].active) {
+          const int n = E.n[lane];
+          v = wave == 0 ? n >> 1 : (n % 2 != 0 && n >= 3) ? 1 : 0;
+        }
+      } else if (lane < G.cells && C[lane].active) {
+        const UnlikeChains &U = C[lane].chains;
+        v = wave == 2 ? U.n : U.big == U.n ? 0 : U.long_chains();
+      }
+      wave_starts(v, lane, pre[wave]);
+    }
+    __syncthreads();
+    for (int stage = 0; stage < STAGES; ++stage) {
+      const int total = pre[stage][64];
+      if (total == 0) continue;
+      for (;;) {
+        uint32_t b = 0;
+        if (lane == 0) b = atomicAdd(&ticket[stage], 64u);
+        const int p = __builtin_amdgcn_readfirstlane((int)b) + lane;
+        if (p - lane >= total) break;
+        // this lane's chain: pairs j0 .. j1 of number k of entry e
+        int e = 0, k = 0, j0 = 0, j1 = 0;
+        if (p < total) {
+          e = entry_of(pre[stage], p);
+          k = p - pre[stage][e];
+          if (stage == 0) j1 = 1;
+          else if (stage == 1) { j0 = 1; j1 = 3; }
+          else {
+            const int len = C[e].chains.length(k);
+            j0 = stage - 2;
+            j1 = stage == 2 ? min(len, 1) : len;
+          }
+        }
+        for (int j = j0; j < j1; ++j) {
+          int cell, sa, sb, ka, kb;
+          uint32_t ord;
+          if (stage < 2) {
+            cell = e >> 1;
+            sa = sb = e & 1;
+            const int n = E.n[e], nel = E.n[2 * cell], nion = E.n[2 * cell + 1];
+            // ordinals in reference order: ion pairs if nion is even, electron
+            // pairs if nel is even, ion pairs if nion is odd, electron pairs if
+            // nel is odd
+            const bool el_first = nion % 2 != 0 && nel % 2 == 0;
+            ord = sa == 0 ? (el_first ? 0 : like_pairs(nion)) : (el_first ? like_pairs(nel) : 0);
+            if (n % 2 == 0) {
+              ka = 2 * k;
+              kb = ka + 1;
+              ord += (uint32_t)k;
+            } else if (k == 0) {
+              // the chain (0, 1), (1, 2), (2, 0)
+              ka = j;
+              kb = j == 2 ? 0 : j + 1;
+              ord += (uint32_t)j;
+            } else {
+              ka = 2 * k + 1;
+              kb = ka + 1;
+              ord += (uint32_t)(k + 2);
+            }
+          } else {
+            cell = e;
+            sa = 0;
+            sb = 1;
+            const int nel = E.n[2 * cell], nion = E.n[2 * cell + 1];
+            const int far = C[cell].chains.partner(k, j);
+            ka = nel <= nion ? k : far;
+            kb = nel <= nion ? far : k;
+            ord = like_pairs(nel) + like_pairs(nion) + (uint32_t)far;
+          }
+          const CellStatsLds &L = C[cell];
+          const int ta = E.start[2 * cell + sa] + ka, tb = E.start[2 * cell + sb] + kb;
+          PairDraws R;
+          const uint64_t ctr = (L.gcell << 24) | (uint64_t)(ord & 0xFFFFFFu);
+          const uint32_t draw = (uint32_t)(2 * step + 1);
+          const double wa = S.w[ta], wb = S.w[tb];
+          uniform2(ctr, draw, seed, R.u[0], R.u[1]);
+          // P12 takes one more, compared with the weights: below them when both are 1 or more
+          R.u[2] = 0;
+          if (SCHEME != COLL_P12 || !(wa >= 1 && wb >= 1)) uniform2(ctr ^ (1ull << 63), draw, seed, R.u[2], R.u[3]);
+          R.pos = 0;
+          double va[3] = {S.vx[ta], S.vy[ta], S.vz[ta]};
+          double vb[3] = {S.vx[tb], S.vy[tb], S.vz[tb]};
+          collide_pair<SCHEME>(sa ? m_i : m_e, sb ? m_i : m_e, sa ? q_i : q_e, sb ? q_i : q_e, va, wa, vb, wb,
+                               L.dens[sa], L.dens[sb], K[SCHEME == COLL_P12 ? cell : 0][sa + sb], L.debye, g.dt, R,
+                               &err);
+          S.vx[ta] = va[0]; S.vy[ta] = va[1]; S.vz[ta] = va[2];
+          S.vx[tb] = vb[0]; S.vy[tb] = vb[1]; S.vz[tb] = vb[2];
+        }
+      }
+      __syncthreads();
     }
     if (SCHEME == COLL_TA77S) {
-      correct_species(S, T, 1, nn[1], m_i, t + 5);
-      correct_species(S, T, 0, nn[0], m_e, t + 0);
+      // correct_velocities runs over every cell
+      __shared__ CorrParams corr[64];
+      if ((int)threadIdx.x < entries) {
+        const int e = threadIdx.x, o = E.start[e];
+        const SlotStage T{S.vx + o, S.vy + o, S.vz + o, S.w + o};
+        corr[e] = correct_params(T, 0, E.n[e], (e & 1) ? m_i : m_e, tot + (long)G.list[e >> 1] * TOT + 5 * (e & 1));
+      }
+      __syncthreads();
+      for (int t = threadIdx.x; t < slots; t += COLL_GROUP_BLOCK) {
+        const CorrParams &P = corr[entry_of(E.start, t)];
+        if (P.ok == 0.0) continue;
+        S.vx[t] = P.V0[0] + P.alpha * (S.vx[t] - P.V0[0] - P.dV[0]);
+        S.vy[t] = P.V0[1] + P.alpha * (S.vy[t] - P.V0[1] - P.dV[1]);
+        S.vz[t] = P.V0[2] + P.alpha * (S.vz[t] - P.V0[2] - P.dV[2]);
+      }
     }
-    for (int k = 0; k < nn[0]; ++k) {
-      double v3[3] = {S.vx(0, k), S.vy(0, k), S.vz(0, k)};
-      ve.store(perm_e[o[0] + k], v3);
+    // every thread stores the slots that it staged (and corrected)
+    for (int t = threadIdx.x; t < slots; t += COLL_GROUP_BLOCK) {
+      const int e = entry_of(E.start, t), k = t - E.start[e];
+      if (k >= E.n[e]) continue;
+      const uint32_t p = ((e & 1) ? perm_i : perm_e)[E.off[e] + k];
+      const double v3[3] = {S.vx[t], S.vy[t], S.vz[t]};
+      if (e & 1) vi.store(p, v3);
+      else ve.store(p, v3);
     }
-    for (int k = 0; k < nn[1]; ++k) {
-      double v3[3] = {S.vx(1, k), S.vy(1, k), S.vz(1, k)};
-      vi.store(perm_i[o[1] + k], v3);
-    }
+    __syncthreads();
   }
   if (err) atomicOr(&st->err, err);
 }
@@ -931,8 +1065,9 @@ __global__ void __launch_bounds__(COLL_CROWD_BLOCK) k_coll_pairs_crowd(
     const double *t = tot + c * TOT;
     if (q.j < row_bad[(long)q.d * g.nr + q.i]) {
       PairRunner<SCHEME, CrowdStage, BlockTeam> P{S, T, {m_e, m_i}, {q_e, q_i}, {t[10], t[11]}, t[12], g.dt, seed,
-                                                  step, (uint64_t)q.cr * (uint64_t)g.Nz + (uint64_t)q.cz, &err,
-                                                  {t[13], t[14]}};
+                                                  step, (uint64_t)q.cr * (uint64_t)g.Nz + (uint64_t)q.cz, &err, {}};
+      if (SCHEME == COLL_P12)
+        for (int k = 0; k < 3; ++k) P.K[k].set_species(k, m_e, m_i, q_e, q_i, t + 10, g.dt);
       cell_pairs(P, nn[0], nn[1]);
     }
     if (SCHEME == COLL_TA77S) {
@@ -1278,13 +1413,10 @@ struct CollBuffers {
   uint32_t *cnt[2] = {nullptr, nullptr}, *off[2] = {nullptr, nullptr};
   uint32_t *fill[2] = {nullptr, nullptr}, *perm[2] = {nullptr, nullptr};
   uint32_t *lists = nullptr, *lcount = nullptr;   // cells per size class
-  double *lane_stage = nullptr;                   // per-lane FP64 stage of the tiny-cell pairs
   uint32_t *crowd_off = nullptr;                  // crowded cells: range of each listed cell
   uint64_t *crowd_key = nullptr;                  // shuffle keys, indices and FP64 stage of
   uint32_t *crowd_idx = nullptr;                  // the crowded cells (COLL_CROWD_CAP particles)
   double *crowd_stage = nullptr;
-  long lane_blocks = 0;
-
   long cap[2] = {0, 0};
   double *tot = nullptr;
   int *row_bad = nullptr;
@@ -1310,7 +1442,7 @@ void coll_free(pcp_ctx *c) {
     (void)hipFree(b->cnt[s]); (void)hipFree(b->off[s]); (void)hipFree(b->fill[s]);
     (void)hipFree(b->perm[s]);
   }
-  (void)hipFree(b->lists); (void)hipFree(b->lcount); (void)hipFree(b->lane_stage);
+  (void)hipFree(b->lists); (void)hipFree(b->lcount);
   (void)hipFree(b->crowd_off); (void)hipFree(b->crowd_key); (void)hipFree(b->crowd_idx); (void)hipFree(b->crowd_stage);
   (void)hipFree(b->tot); (void)hipFree(b->row_bad); (void)hipFree(b->scan_tmp);
   (void)hipFree(b->mom); (void)hipFree(b->mom2); (void)hipFree(b->feat); (void)hipFree(b->pred);
@@ -1337,16 +1469,12 @@ static int coll_alloc(pcp_ctx *c, long cap_e, long cap_i) {
         hipMalloc(&b->perm[s], caps[s] * sizeof(uint32_t)) != hipSuccess)
       return -1;
   }
-  // the lane-per-cell kernels: four workgroups per CU, COLL_LANE_SLOTS doubles per lane
-  b->lane_blocks = (long)c->n_cu * 4;
   if (hipMalloc(&b->lists, (size_t)COLL_CLASSES * ncells * sizeof(uint32_t)) != hipSuccess ||
       hipMalloc(&b->lcount, (COLL_CLASSES + 1) * sizeof(uint32_t)) != hipSuccess ||
       hipMalloc(&b->crowd_off, COLL_CROWD_CELLS * sizeof(uint32_t)) != hipSuccess ||
       hipMalloc(&b->crowd_key, COLL_CROWD_CAP * sizeof(uint64_t)) != hipSuccess ||
       hipMalloc(&b->crowd_idx, COLL_CROWD_CAP * sizeof(uint32_t)) != hipSuccess ||
-      hipMalloc(&b->crowd_stage, 4 * COLL_CROWD_CAP * sizeof(double)) != hipSuccess ||
-      hipMalloc(&b->lane_stage, (size_t)COLL_LANE_SLOTS * b->lane_blocks * COLL_LANE_BLOCK * sizeof(double)) !=
-          hipSuccess)
+      hipMalloc(&b->crowd_stage, 4 * COLL_CROWD_CAP * sizeof(double)) != hipSuccess)
     return -1;
   if (hipMalloc(&b->tot, ncells * TOT * sizeof(double)) != hipSuccess ||
       hipMalloc(&b->row_bad, (long)c->D * c->g.nr * sizeof(int)) != hipSuccess ||
@@ -1398,70 +1526,36 @@ static int coll_buckets(pcp_ctx *c, V ve, V vi, long n_e, long n_i, const int *m
   return 0;
 }
 
-// the binary pass (shuffle + statistics, then pairs) on the cells of `mask`
-// (all cells when null)
-template <class V, int CLS>
-static void coll_class(pcp_ctx *c, int scheme, V ve, V vi, double m_e, double m_i, double q_e, double q_i,
-                       uint64_t seed, PassNo step, bool pairs, const unsigned long long *gate) {
+// shuffle and statistics of every listed cell: the grouped classes in one
+// launch, the crowded cells in another
+template <class V>
+static void coll_prep(pcp_ctx *c, V ve, V vi, double m_e, double m_i, uint64_t seed, PassNo step,
+                      const unsigned long long *gate) {
   CollBuffers *b = c->coll;
   const Geom &g = c->g;
-  constexpr int MAXC = COLL_CLASS_MAXC[CLS];
-  const uint32_t *list = b->lists + (size_t)CLS * b->ncells, *count = b->lcount + CLS;
-  const unsigned gc = (unsigned)std::min<long>(b->ncells, (long)c->n_cu * 32);
-  if constexpr (CLS == 0) {
-    const unsigned gl = (unsigned)b->lane_blocks;
-    if (!pairs)
-      hipLaunchKernelGGL((k_coll_prep_lane<V>), dim3(gl), dim3(COLL_LANE_BLOCK), 0, c->stream, g, ve, vi, b->off[0],
-                         b->off[1], b->perm[0], b->perm[1], m_e, m_i, seed, step, b->tot, b->row_bad, list, count,
-                         gate);
-    else if (scheme == COLL_TA77S)
-      hipLaunchKernelGGL((k_coll_pairs_lane<COLL_TA77S, V>), dim3(gl), dim3(COLL_LANE_BLOCK), 0, c->stream, g, ve,
-                         vi, b->off[0], b->off[1], b->perm[0], b->perm[1], m_e, m_i, q_e, q_i, seed, step, b->tot,
-                         b->row_bad, list, count, b->lane_stage, c->st, gate);
-    else if (scheme == COLL_SK98)
-      hipLaunchKernelGGL((k_coll_pairs_lane<COLL_SK98, V>), dim3(gl), dim3(COLL_LANE_BLOCK), 0, c->stream, g, ve,
-                         vi, b->off[0], b->off[1], b->perm[0], b->perm[1], m_e, m_i, q_e, q_i, seed, step, b->tot,
-                         b->row_bad, list, count, b->lane_stage, c->st, gate);
-    else
-      hipLaunchKernelGGL((k_coll_pairs_lane<COLL_P12, V>), dim3(gl), dim3(COLL_LANE_BLOCK), 0, c->stream, g, ve,
-                         vi, b->off[0], b->off[1], b->perm[0], b->perm[1], m_e, m_i, q_e, q_i, seed, step, b->tot,
-                         b->row_bad, list, count, b->lane_stage, c->st, gate);
-  } else if constexpr (CLS == COLL_CLASSES - 1) {
-    const unsigned gw = (unsigned)(c->n_cu * 2);
-    if (!pairs)
-      hipLaunchKernelGGL((k_coll_prep_crowd<V>), dim3(gw), dim3(COLL_CROWD_BLOCK), 0, c->stream, g, ve, vi,
-                         b->off[0], b->off[1], b->perm[0], b->perm[1], m_e, m_i, seed, step, b->tot, b->row_bad,
-                         list, count, b->crowd_off, b->crowd_key, b->crowd_idx, b->crowd_stage, gate);
-    else if (scheme == COLL_TA77S)
-      hipLaunchKernelGGL((k_coll_pairs_crowd<COLL_TA77S, V>), dim3(gw), dim3(COLL_CROWD_BLOCK), 0, c->stream, g, ve,
-                         vi, b->off[0], b->off[1], b->perm[0], b->perm[1], m_e, m_i, q_e, q_i, seed, step, b->tot,
-                         b->row_bad, list, count, b->crowd_off, b->crowd_stage, c->st, gate);
-    else if (scheme == COLL_SK98)
-      hipLaunchKernelGGL((k_coll_pairs_crowd<COLL_SK98, V>), dim3(gw), dim3(COLL_CROWD_BLOCK), 0, c->stream, g, ve,
-                         vi, b->off[0], b->off[1], b->perm[0], b->perm[1], m_e, m_i, q_e, q_i, seed, step, b->tot,
-                         b->row_bad, list, count, b->crowd_off, b->crowd_stage, c->st, gate);
-    else
-      hipLaunchKernelGGL((k_coll_pairs_crowd<COLL_P12, V>), dim3(gw), dim3(COLL_CROWD_BLOCK), 0, c->stream, g, ve,
-                         vi, b->off[0], b->off[1], b->perm[0], b->perm[1], m_e, m_i, q_e, q_i, seed, step, b->tot,
-                         b->row_bad, list, count, b->crowd_off, b->crowd_stage, c->st, gate);
-  } else {
-  if (!pairs)
-    hipLaunchKernelGGL((k_coll_prep<V, MAXC>), dim3(gc), dim3(COLL_BLOCK), 0, c->stream, g, ve, vi, b->off[0],
-                       b->off[1], b->perm[0], b->perm[1], m_e, m_i, seed, step, b->tot, b->row_bad, list, count, c->st,
-                       gate);
-  else if (scheme == COLL_TA77S)
-    hipLaunchKernelGGL((k_coll_pairs<COLL_TA77S, V, MAXC>), dim3(gc), dim3(COLL_BLOCK), 0, c->stream, g, ve, vi,
-                       b->off[0], b->off[1], b->perm[0], b->perm[1], m_e, m_i, q_e, q_i, seed, step, b->tot,
-                       b->row_bad, list, count, c->st, gate);
-  else if (scheme == COLL_SK98)
-    hipLaunchKernelGGL((k_coll_pairs<COLL_SK98, V, MAXC>), dim3(gc), dim3(COLL_BLOCK), 0, c->stream, g, ve, vi,
-                       b->off[0], b->off[1], b->perm[0], b->perm[1], m_e, m_i, q_e, q_i, seed, step, b->tot,
-                       b->row_bad, list, count, c->st, gate);
-  else
-    hipLaunchKernelGGL((k_coll_pairs<COLL_P12, V, MAXC>), dim3(gc), dim3(COLL_BLOCK), 0, c->stream, g, ve, vi,
-                       b->off[0], b->off[1], b->perm[0], b->perm[1], m_e, m_i, q_e, q_i, seed, step, b->tot,
-                       b->row_bad, list, count, c->st, gate);
-  }
+  hipLaunchKernelGGL((k_coll_prep<V>), dim3((unsigned)c->n_cu * 12), dim3(COLL_GROUP_BLOCK), 0, c->stream, g, ve, vi,
+                     b->off[0], b->off[1], b->perm[0], b->perm[1], m_e, m_i, seed, step, b->tot, b->lists,
+                     b->lcount, b->ncells, gate);
+  hipLaunchKernelGGL(k_coll_stats, dim3((unsigned)std::max(1L, std::min<long>((b->ncells + 255) / 256, (long)c->n_cu * 8))),
+                     dim3(256), 0, c->stream, g, b->tot, b->row_bad, b->lists, b->lcount, b->ncells, gate);
+  hipLaunchKernelGGL((k_coll_prep_crowd<V>), dim3((unsigned)c->n_cu * 2), dim3(COLL_CROWD_BLOCK), 0, c->stream, g, ve,
+                     vi, b->off[0], b->off[1], b->perm[0], b->perm[1], m_e, m_i, seed, step, b->tot, b->row_bad,
+                     b->lists + (size_t)COLL_GROUP_CLASSES * b->ncells, b->lcount + COLL_GROUP_CLASSES, b->crowd_off,
+                     b->crowd_key, b->crowd_idx, b->crowd_stage, gate);
+}
+
+template <int SCHEME, class V>
+static void coll_pairs(pcp_ctx *c, V ve, V vi, double m_e, double m_i, double q_e, double q_i, uint64_t seed,
+                       PassNo step, const unsigned long long *gate) {
+  CollBuffers *b = c->coll;
+  const Geom &g = c->g;
+  hipLaunchKernelGGL((k_coll_pairs<SCHEME, V>), dim3((unsigned)c->n_cu * 8), dim3(COLL_GROUP_BLOCK), 0, c->stream, g,
+                     ve, vi, b->off[0], b->off[1], b->perm[0], b->perm[1], m_e, m_i, q_e, q_i, seed, step, b->tot,
+                     b->row_bad, b->lists, b->lcount, b->ncells, c->st, gate);
+  hipLaunchKernelGGL((k_coll_pairs_crowd<SCHEME, V>), dim3((unsigned)c->n_cu * 2), dim3(COLL_CROWD_BLOCK), 0,
+                     c->stream, g, ve, vi, b->off[0], b->off[1], b->perm[0], b->perm[1], m_e, m_i, q_e, q_i, seed,
+                     step, b->tot, b->row_bad, b->lists + (size_t)COLL_GROUP_CLASSES * b->ncells,
+                     b->lcount + COLL_GROUP_CLASSES, b->crowd_off, b->crowd_stage, c->st, gate);
 }
 
 // the binary pass on the cells of `mask` (all cells when null): cells
@@ -1480,14 +1574,10 @@ static void coll_binary(pcp_ctx *c, int scheme, V ve, V vi, double m_e, double m
   const unsigned gz = (unsigned)std::max(1L, std::min<long>((ncells + 255) / 256, (long)c->n_cu * 16));
   hipLaunchKernelGGL(k_coll_classify, dim3(gz), dim3(256), 0, c->stream, g, b->off[0], b->off[1], mask, b->lists,
                      b->lcount, b->crowd_off, b->row_bad, c->st, gate);
-  coll_class<V, 0>(c, scheme, ve, vi, m_e, m_i, q_e, q_i, seed, step, false, gate);
-  coll_class<V, 1>(c, scheme, ve, vi, m_e, m_i, q_e, q_i, seed, step, false, gate);
-  coll_class<V, 2>(c, scheme, ve, vi, m_e, m_i, q_e, q_i, seed, step, false, gate);
-  coll_class<V, 3>(c, scheme, ve, vi, m_e, m_i, q_e, q_i, seed, step, false, gate);
-  coll_class<V, 0>(c, scheme, ve, vi, m_e, m_i, q_e, q_i, seed, step, true, gate);
-  coll_class<V, 1>(c, scheme, ve, vi, m_e, m_i, q_e, q_i, seed, step, true, gate);
-  coll_class<V, 2>(c, scheme, ve, vi, m_e, m_i, q_e, q_i, seed, step, true, gate);
-  coll_class<V, 3>(c, scheme, ve, vi, m_e, m_i, q_e, q_i, seed, step, true, gate);
+  coll_prep(c, ve, vi, m_e, m_i, seed, step, gate);
+  if (scheme == COLL_TA77S) coll_pairs<COLL_TA77S>(c, ve, vi, m_e, m_i, q_e, q_i, seed, step, gate);
+  else if (scheme == COLL_SK98) coll_pairs<COLL_SK98>(c, ve, vi, m_e, m_i, q_e, q_i, seed, step, gate);
+  else coll_pairs<COLL_P12>(c, ve, vi, m_e, m_i, q_e, q_i, seed, step, gate);
 }
 
 template <class V>
