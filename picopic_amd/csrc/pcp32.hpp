@@ -46,14 +46,29 @@ struct SortBuffers32 {
   uint64_t *seq, *id;
 };
 
+// Cell and FP32 in-cell offset of a coordinate u (cell units) of a grid of n
+// cells.  An offset that rounds to 1 moves to the next cell -- at the last cell
+// it stays at the largest offset below 1: the cell past it is outside the grid.
+__host__ __device__ __forceinline__ void split_coordinate(double u, long n, long &cell, float &f) {
+  const double fc = floor(u);
+  cell = (long)fc;
+  f = (float)(u - fc);
+  if (f >= 1.f) {
+    f = 0.f;
+    cell += 1;
+  }
+  if (cell >= n) {
+    cell = n - 1;
+    f = 1.f - 0x1p-24f;
+  }
+}
+
 // position (r, z) in split form, written to both position slots of q
 __device__ __forceinline__ void store_split(Species32 &s, long q, const Geom &g, double r, double z) {
-  double ur = r / g.dr, uz = z / g.dz;
-  double fcr = floor(ur), fcz = floor(uz);
-  float fr = (float)(ur - fcr), fz = (float)(uz - fcz);
-  int cr = (int)fcr, cz = (int)fcz;
-  if (fr >= 1.f) { fr = 0.f; cr += 1; }
-  if (fz >= 1.f) { fz = 0.f; cz += 1; }
+  long cr, cz;
+  float fr, fz;
+  split_coordinate(r / g.dr, g.Nr, cr, fr);
+  split_coordinate(z / g.dz, g.Nz, cz, fz);
   uint32_t cell = (uint32_t)cr * (uint32_t)g.Nz + (uint32_t)cz;
   s.cell[0][q] = cell; s.cell[1][q] = cell;
   s.fr[0][q] = fr; s.fr[1][q] = fr;

@@ -438,13 +438,10 @@ int pcp_upload_species(pcp_ctx *c, int sp, long n, const double *r, const double
     std::vector<uint32_t> cell(n);
     std::vector<float> fr(n), fz(n), fvr(n), fvp(n), fvz(n), fw(n);
     for (long p = 0; p < n; ++p) {
-      double ur = r[p] / g.dr, uz = z[p] / g.dz;
-      double ir = std::floor(ur), iz = std::floor(uz);
-      float a = (float)(ur - ir), b = (float)(uz - iz);
-      if (a >= 1.f) { a = 0.f; ir += 1; }
-      if (b >= 1.f) { b = 0.f; iz += 1; }
-      cell[p] = (uint32_t)((long)ir * g.Nz + (long)iz);
-      fr[p] = a; fz[p] = b;
+      long ir, iz;
+      split_coordinate(r[p] / g.dr, g.Nr, ir, fr[p]);
+      split_coordinate(z[p] / g.dz, g.Nz, iz, fz[p]);
+      cell[p] = (uint32_t)(ir * g.Nz + iz);
       fvr[p] = (float)vr[p]; fvp[p] = (float)vphi[p]; fvz[p] = (float)vz[p]; fw[p] = (float)w[p];
     }
     size_t off = (size_t)s.n, fb = (size_t)n * sizeof(float);

@@ -1,0 +1,45 @@
+"""FP32 split positions next to the outer edges of the grid.
+
+A coordinate within 2^-25 of a cell below the grid's end has an in-cell offset
+that rounds to 1, which must not carry it into the cell past the last one (the
+sort's counters and the field grids end there).
+"""
+import numpy as np
+import pytest
+
+from picopic_amd import capi
+
+pytestmark = pytest.mark.gpu
+
+CELL = 1e-3
+
+
+def check(ctx, grid):
+    p = ctx.particles(0)
+    assert (p["r"] < grid[0] * CELL).all() and (p["z"] < grid[1] * CELL).all()
+    return p
+
+
+@pytest.mark.parametrize("domains", [(1, 1), (2, 2)])
+def test_uploaded_particles_stay_in_the_last_cell(domains):
+    grid = (8, 16)
+    ctx = capi.Context((grid[0] * CELL, grid[1] * CELL), grid, domains, 1e-13, [(-1, 1, False, 64)], precision="fp32")
+    u = np.array([[8 - 1e-9, 5.5], [7.5, 16 - 1e-9], [8 - 1e-9, 16 - 1e-9], [3 - 1e-9, 4.5], [2.25, 3.125]])
+    z = np.zeros(len(u))
+    ctx.upload(0, u[:, 0] * CELL, u[:, 1] * CELL, z, z, z, z + 1e6)
+    print("upload", domains, flush=True)
+    p = check(ctx, grid)
+    # positions keep 2^-24 of a cell
+    assert np.abs(p["r"] / CELL - u[:, 0]).max() <= 2.0 ** -23
+    assert np.abs(p["z"] / CELL - u[:, 1]).max() <= 2.0 ** -23
+
+
+def test_initial_plasma_stays_in_the_last_cell():
+    # with this seed particle 40689 of the outer row lies at r / dr = 2 - 2e-8
+    grid = (2, 2)
+    ctx = capi.Context((grid[0] * CELL, grid[1] * CELL), grid, (1, 1), 1e-13, [(-1, 1, False, 100000)],
+                       precision="fp32")
+    ctx.init_plasma(0, 20000, 1e17, 1e17, 1.0, 1427)
+    print("init_plasma", flush=True)
+    p = check(ctx, grid)
+    assert len(p["r"]) == 80000 and p["r"].max() > (2 - 1e-6) * CELL
