@@ -181,8 +181,12 @@ __host__ __device__ inline double *ehist_row(double *h, unsigned long long step)
   return h + (long)(step % EHIST) * EHIST_COLS;
 }
 
-// domain owning global cell (cr, cz)
-__device__ __forceinline__ int domain_of(const Geom &g, int cr, int cz) { return (cr / g.nr) * g.Dz + (cz / g.nz); }
+// domain owning global cell (cr, cz) (a cell below the grid, which a particle
+// that is not collected yet can be in, divides toward zero)
+__device__ __forceinline__ int domain_of(const Geom &g, int cr, int cz) {
+  if ((cr | cz) >= 0) return (int)g.div_nr.div((uint32_t)cr) * g.Dz + (int)g.div_nz.div((uint32_t)cz);
+  return (cr / g.nr) * g.Dz + (cz / g.nz);
+}
 
 // Appends particle p of species sp, moving from domain d_old to d_new, to
 // the step's migrant list.  Its key orders the arrivals of a destination as

@@ -314,9 +314,9 @@ __device__ __forceinline__ bool move_one(const Geom &g, int beam, double &r, dou
   move_particle(g, dm, beam, r, z, vr, vphi, vz, vzo);
   vz = vzo;
   if (bad_position(r, z)) return false;
-  long cr = (long)floor(r / g.dr), cz = (long)floor(z / g.dz);
+  const int cr = cell_number(r, g.dr), cz = cell_number(z, g.dz);
   if (cr < 0 || cz < 0 || cr >= g.Nr || cz >= g.Nz) return false;
-  d_new = domain_of(g, (int)cr, (int)cz);
+  d_new = domain_of(g, cr, cz);
   return true;
 }
 
