@@ -99,11 +99,22 @@ struct GridView32 {
   }
 };
 
-// E (maxwellSolver.hpp:211-316) in cell units
-__device__ __forceinline__ void gather32_e(const GridView32 &E, int cr, int cz, float fr, float fz, float out[3]) {
+// the weights and nodes of a position, the same for E and H (they are formed
+// once: the compiler does not merge two copies over rad_half's branches)
+struct GatherWeights32 {
+  W2 ra, ri;
+  Z2 zi, zh;
+};
+__device__ __forceinline__ GatherWeights32 gather_weights32(int cr, int cz, float fr, float fz) {
 #pragma clang fp contract(fast)
-  W2 ra = rad_half(cr, fr), ri = rad_int(cr, fr);
-  Z2 zi = z_int(cz, fz), zh = z_half(cz, fz);
+  return GatherWeights32{rad_half(cr, fr), rad_int(cr, fr), z_int(cz, fz), z_half(cz, fz)};
+}
+
+// E (maxwellSolver.hpp:211-316) in cell units
+__device__ __forceinline__ void gather32_e(const GridView32 &E, const GatherWeights32 &w, float out[3]) {
+#pragma clang fp contract(fast)
+  const W2 ra = w.ra, ri = w.ri;
+  const Z2 zi = w.zi, zh = w.zh;
   float c0 = 0.f, c1 = 0.f, c2 = 0.f;
   // E_r: node (floor(u - 1/2), floor(w))
   c0 += E.at(0, ra.i, zi.k) * (ra.a1 * zi.w1);
@@ -124,10 +135,10 @@ __device__ __forceinline__ void gather32_e(const GridView32 &E, int cr, int cz, 
 }
 
 // H (maxwellSolver.hpp:101-209) in cell units
-__device__ __forceinline__ void gather32_h(const GridView32 &H, int cr, int cz, float fr, float fz, float out[3]) {
+__device__ __forceinline__ void gather32_h(const GridView32 &H, const GatherWeights32 &w, float out[3]) {
 #pragma clang fp contract(fast)
-  W2 ra = rad_half(cr, fr), ri = rad_int(cr, fr);
-  Z2 zi = z_int(cz, fz), zh = z_half(cz, fz);
+  const W2 ra = w.ra, ri = w.ri;
+  const Z2 zi = w.zi, zh = w.zh;
   float c0 = 0.f, c1 = 0.f, c2 = 0.f;
   // H_z: node (floor(u - 1/2), floor(w))
   c2 += H.at(2, ra.i, zi.k) * (ra.a1 * zi.w1);
@@ -181,31 +192,42 @@ __device__ __forceinline__ void apply_cell_rescale(const float *cpar, int cslot,
   v[2] = Vz + az * (v[2] - Vz);
 }
 
-__device__ __forceinline__ float len2f(const float v[3]) { return v[0] * v[0] + v[1] * v[1] + v[2] * v[2]; }
+__device__ __forceinline__ float dot3f(const float a[3], const float b[3]) {
+  return __builtin_fmaf(a[2], b[2], __builtin_fmaf(a[1], b[1], a[0] * b[0]));
+}
+__device__ __forceinline__ float len2f(const float v[3]) { return dot3f(v, v); }
 
+// The sums of products are written as FMAs (explicitly: every kernel that
+// pushes has to round alike), a rounding less each and two thirds of the
+// instructions.  With the run sums' multiply-adds (pcp_wave.hpp) the
+// push of the full form took 553 -> 383 vector instructions a wavefront of
+// 64 particles (4.49 -> 3.99 ms for 2.7e8 particles), the VB step 11 % less
+// time (4.71 -> 4.20 ms for 1.5e8).
 __device__ __forceinline__ void push32(int pusher, const PushConst &K, float e[3], float b[3], float v[3], int *err) {
+#define FMA __builtin_fmaf
   if (pusher <= PCP_PUSHER_BORIS_ADAPTIVE) {
     const bool rel = pusher != PCP_PUSHER_BORIS;
-    for (int i = 0; i < 3; ++i) { e[i] *= K.c2m; b[i] *= K.c2m_mu; }
+    float bs = K.c2m_mu;
     if (rel) {
       float beta = len2f(v) * K.inv_c2;
       if (beta > 1.f) *err |= ERR_BETA_GT_1;
       float gamma = rsqrt_f(1.f - beta);
       for (int i = 0; i < 3; ++i) v[i] *= gamma;
     }
-    for (int i = 0; i < 3; ++i) v[i] += e[i];
-    if (rel) {
-      float gi = rsqrt_f(1.f + len2f(v) * K.inv_c2);
-      for (int i = 0; i < 3; ++i) b[i] *= gi;
-    }
+    for (int i = 0; i < 3; ++i) v[i] = FMA(e[i], K.c2m, v[i]);
+    if (rel) bs *= rsqrt_f(FMA(len2f(v), K.inv_c2, 1.f));
+    for (int i = 0; i < 3; ++i) b[i] *= bs;
     float const2 = 2.f * rcp_f(1.f + len2f(b));
-    float t0 = v[0], t1 = v[1], t2 = v[2];
-    v[0] = t0 + const2 * ((t1 - t0 * b[2] + t2 * b[0]) * b[2] - (t2 + t0 * b[1] - t1 * b[0]) * b[1]);
-    v[1] = t1 + const2 * (-(t0 + t1 * b[2] - t2 * b[1]) * b[2] + (t2 + t0 * b[1] - t1 * b[0]) * b[0]);
-    v[2] = t2 + const2 * ((t0 + t1 * b[2] - t2 * b[1]) * b[1] - (t1 - t0 * b[2] + t2 * b[0]) * b[0]);
-    for (int i = 0; i < 3; ++i) v[i] += e[i];
+    const float t0 = v[0], t1 = v[1], t2 = v[2];
+    const float u1 = FMA(t2, b[0], FMA(-t0, b[2], t1));
+    const float u2 = FMA(-t1, b[0], FMA(t0, b[1], t2));
+    const float u0 = FMA(-t2, b[1], FMA(t1, b[2], t0));
+    v[0] = FMA(const2, FMA(u1, b[2], -(u2 * b[1])), t0);
+    v[1] = FMA(const2, FMA(u2, b[0], -(u0 * b[2])), t1);
+    v[2] = FMA(const2, FMA(u0, b[1], -(u1 * b[0])), t2);
+    for (int i = 0; i < 3; ++i) v[i] = FMA(e[i], K.c2m, v[i]);
     if (rel) {
-      float gi = rsqrt_f(1.f + len2f(v) * K.inv_c2);
+      float gi = rsqrt_f(FMA(len2f(v), K.inv_c2, 1.f));
       for (int i = 0; i < 3; ++i) v[i] *= gi;
     }
   } else if (pusher == PCP_PUSHER_VAY) {
@@ -214,51 +236,53 @@ __device__ __forceinline__ void push32(int pusher, const PushConst &K, float e[3
     float gamma = rsqrt_f(1.f - beta);
     for (int i = 0; i < 3; ++i) v[i] *= gamma;
     float up[3];
-    for (int i = 0; i < 3; ++i) { up[i] = v[i] + e[i] * (2.f * K.c2m); b[i] *= K.c2m_mu; }
-    float gi = rsqrt_f(1.f + len2f(v) * K.inv_c2);
-    up[0] += gi * (v[1] * b[2] - v[2] * b[1]);
-    up[1] += gi * (v[2] * b[0] - v[0] * b[2]);
-    up[2] += gi * (v[0] * b[1] - v[1] * b[0]);
+    for (int i = 0; i < 3; ++i) { up[i] = FMA(e[i], 2.f * K.c2m, v[i]); b[i] *= K.c2m_mu; }
+    float gi = rsqrt_f(FMA(len2f(v), K.inv_c2, 1.f));
+    up[0] = FMA(gi, FMA(v[1], b[2], -(v[2] * b[1])), up[0]);
+    up[1] = FMA(gi, FMA(v[2], b[0], -(v[0] * b[2])), up[1]);
+    up[2] = FMA(gi, FMA(v[0], b[1], -(v[1] * b[0])), up[2]);
     float alpha = 1.f + len2f(up);   // unit mix of the reference (quirk Q4)
     float B2 = len2f(b);
     float s = alpha - B2;
-    float ub = up[0] * b[0] + up[1] * b[1] + up[2] * b[2];
-    alpha = rsqrt_f(0.5f * (s + sqrt_f(s * s + 4.f * (B2 + ub * ub))));
+    float ub = dot3f(up, b);
+    alpha = rsqrt_f(0.5f * (s + sqrt_f(FMA(s, s, 4.f * FMA(ub, ub, B2)))));
     for (int i = 0; i < 3; ++i) b[i] *= alpha;
     s = rcp_f(1.f + len2f(b));
-    alpha = up[0] * b[0] + up[1] * b[1] + up[2] * b[2];
+    alpha = dot3f(up, b);
     float psm[3];
-    psm[0] = s * (up[0] + alpha * b[0] + b[2] * up[1] - b[1] * up[2]);
-    psm[1] = s * (up[1] + alpha * b[1] + b[0] * up[2] - b[2] * up[0]);
-    psm[2] = s * (up[2] + alpha * b[2] + b[1] * up[0] - b[0] * up[1]);
-    gi = rsqrt_f(1.f + len2f(psm) * K.inv_c2);
+    psm[0] = s * FMA(-b[1], up[2], FMA(b[2], up[1], FMA(alpha, b[0], up[0])));
+    psm[1] = s * FMA(-b[2], up[0], FMA(b[0], up[2], FMA(alpha, b[1], up[1])));
+    psm[2] = s * FMA(-b[0], up[1], FMA(b[1], up[0], FMA(alpha, b[2], up[2])));
+    gi = rsqrt_f(FMA(len2f(psm), K.inv_c2, 1.f));
     for (int i = 0; i < 3; ++i) v[i] = psm[i] * gi;
   } else {
     float beta = len2f(v) * K.inv_c2;
     if (beta > 1.f) *err |= ERR_BETA_GT_1;
     float gamma = rsqrt_f(1.f - beta);
-    float um[3], psm[3], b2[3], bc[3], up[3];
+    float um[3], psm[3], b2[3], up[3];
     for (int i = 0; i < 3; ++i) {
-      v[i] *= gamma;
       psm[i] = e[i] * K.c2m;
-      um[i] = v[i] + psm[i];
+      um[i] = FMA(v[i], gamma, psm[i]);
       b[i] *= K.c2m_mu;
     }
     float gfm2 = 1.f + len2f(um);   // quirk Q5
     float B2 = len2f(b);
-    float bu = b[0] * um[0] + b[1] * um[1] + b[2] * um[2];
+    float bu = dot3f(b, um);
     float gb = gfm2 - B2;
-    gamma = rsqrt_f(0.5f * (gb + sqrt_f(gb * gb + 4.f * (B2 + bu * bu))));
+    gamma = rsqrt_f(0.5f * (gb + sqrt_f(FMA(gb, gb, 4.f * FMA(bu, bu, B2)))));
     for (int i = 0; i < 3; ++i) { b[i] *= gamma; b2[i] = b[i] * b[i]; }
-    bc[0] = b[0] * b[1]; bc[1] = b[1] * b[2]; bc[2] = b[2] * b[0];
     float inv_det_B = rcp_f(1.f + b2[0] + b2[1] + b2[0]);   // b2[0] twice (pusherHC.cpp:94)
-    up[0] = ((1.f + b2[0] - b2[1] - b2[2]) * um[0] + 2.f * (bc[0] + b[2]) * um[1] + 2.f * (bc[2] - b[2]) * um[2]) * inv_det_B;
-    up[1] = (2.f * (bc[0] - b[2]) * um[0] + (1.f - b2[0] + b2[1] - b2[2]) * um[1] + 2.f * (bc[1] + b[0]) * um[2]) * inv_det_B;
-    up[2] = (2.f * (bc[2] + b[1]) * um[0] + 2.f * (bc[1] - b[0]) * um[1] + (1.f - b2[0] - b2[1] + b2[2]) * um[2]) * inv_det_B;
-    for (int i = 0; i < 3; ++i) psm[i] += up[i];
-    float gi = rsqrt_f(1.f + len2f(psm) * K.inv_c2);
+    up[0] = FMA(2.f, FMA(FMA(b[0], b[1], b[2]), um[1], FMA(b[2], b[0], -b[2]) * um[2]),
+                (1.f + b2[0] - b2[1] - b2[2]) * um[0]);
+    up[1] = FMA(2.f, FMA(FMA(b[0], b[1], -b[2]), um[0], FMA(b[1], b[2], b[0]) * um[2]),
+                (1.f - b2[0] + b2[1] - b2[2]) * um[1]);
+    up[2] = FMA(2.f, FMA(FMA(b[2], b[0], b[1]), um[0], FMA(b[1], b[2], -b[0]) * um[1]),
+                (1.f - b2[0] - b2[1] + b2[2]) * um[2]);
+    for (int i = 0; i < 3; ++i) psm[i] = FMA(up[i], inv_det_B, psm[i]);
+    float gi = rsqrt_f(FMA(len2f(psm), K.inv_c2, 1.f));
     for (int i = 0; i < 3; ++i) v[i] = psm[i] * gi;
   }
+#undef FMA
 }
 
 // ---------------------------------------------------------------------------
@@ -457,8 +481,9 @@ __device__ __forceinline__ bool advance32(const Geom &g, const FieldsT<float> &f
     GridView32 EV{f.E + (long)d_old * 3 * g.P, g.P, g.yr, dm.bot_r, dm.left_z};
     GridView32 HV{f.H + (long)d_old * 3 * g.P, g.P, g.yr, dm.bot_r, dm.left_z};
     float e[3], h[3];
-    gather32_e(EV, o.cr, o.cz, o.fr, o.fz, e);
-    gather32_h(HV, o.cr, o.cz, o.fr, o.fz, h);
+    const GatherWeights32 gw = gather_weights32(o.cr, o.cz, o.fr, o.fz);
+    gather32_e(EV, gw, e);
+    gather32_h(HV, gw, h);
     push32(g.pusher, K, e, h, v, err);
   }
   n = o;
@@ -480,8 +505,9 @@ __global__ void __launch_bounds__(256) k32_push(Geom g, FieldsT<float> f, Specie
     GridView32 EV{f.E + (long)d * 3 * g.P, g.P, g.yr, dm.bot_r, dm.left_z};
     GridView32 HV{f.H + (long)d * 3 * g.P, g.P, g.yr, dm.bot_r, dm.left_z};
     float e[3], h[3];
-    gather32_e(EV, o.cr, o.cz, o.fr, o.fz, e);
-    gather32_h(HV, o.cr, o.cz, o.fr, o.fz, h);
+    const GatherWeights32 gw = gather_weights32(o.cr, o.cz, o.fr, o.fz);
+    gather32_e(EV, gw, e);
+    gather32_h(HV, gw, h);
     float v[3] = {s.vr[cur][p], s.vphi[cur][p], s.vz[cur][p]};
     push32(g.pusher, K, e, h, v, &err);
     s.vr[nxt][p] = v[0]; s.vphi[nxt][p] = v[1]; s.vz[nxt][p] = v[2];
@@ -495,9 +521,15 @@ __global__ void __launch_bounds__(256) k32_push(Geom g, FieldsT<float> f, Specie
 // sum w, sum w v (r, phi, z), sum w v_z^2, sum w (v_r^2 + v_phi^2) -- the
 // sums behind the surrogate's temperatures.  A wavefront takes 64
 // consecutive (cell-ordered) particles; the lanes of a cell form runs whose
-// sums (DPP run sums in FP32) leave one FP64 atomic per run and moment.
+// sums (DPP run sums in FP32) leave one FP64 atomic per run and moment.  The
+// sums of eight runs pass through LDS to one atomic instruction: eight lanes
+// a run, so that a run's seven atomics hit one cache line (seven instructions
+// with one lane per run each cost 2.3 ms more per full-form step: the L2 takes
+// same-line lanes of an instruction together).
 __global__ void __launch_bounds__(256) k32_push_mom(Geom g, FieldsT<float> f, Species32 s, int cur, StepState *st,
                                                     PushConst K, double *mom, int slot) {
+  __shared__ __align__(16) float run_rows[4][8][8];
+  float(*const run)[8] = run_rows[threadIdx.x >> 6];
   int err = 0;
   const int nxt = cur ^ 1;
   const int lane = threadIdx.x & 63;
@@ -516,8 +548,9 @@ __global__ void __launch_bounds__(256) k32_push_mom(Geom g, FieldsT<float> f, Sp
         GridView32 EV{f.E + (long)d * 3 * g.P, g.P, g.yr, dm.bot_r, dm.left_z};
         GridView32 HV{f.H + (long)d * 3 * g.P, g.P, g.yr, dm.bot_r, dm.left_z};
         float e[3], h[3];
-        gather32_e(EV, o.cr, o.cz, o.fr, o.fz, e);
-        gather32_h(HV, o.cr, o.cz, o.fr, o.fz, h);
+        const GatherWeights32 gw = gather_weights32(o.cr, o.cz, o.fr, o.fz);
+        gather32_e(EV, gw, e);
+        gather32_h(HV, gw, h);
         v[0] = s.vr[cur][p]; v[1] = s.vphi[cur][p]; v[2] = s.vz[cur][p];
         push32(g.pusher, K, e, h, v, &err);
         s.vr[nxt][p] = v[0]; s.vphi[nxt][p] = v[1]; s.vz[nxt][p] = v[2];
@@ -530,25 +563,29 @@ __global__ void __launch_bounds__(256) k32_push_mom(Geom g, FieldsT<float> f, Sp
       const bool live = key != DEAD_CELL;
       float q[7] = {live ? 1.f : 0.f, w, w * v[0], w * v[1], w * v[2], w * v[2] * v[2],
                     w * (v[0] * v[0] + v[1] * v[1])};
+      if (run_sums_bounded(q)) {
+        run_sums_f(q[0], q[1], q[2], q[3], R);
+        run_sums_f(q[4], q[5], q[6], R);
+      } else {
 #pragma unroll
-      for (int k = 0; k < 7; ++k) q[k] = run_sum_f(q[k], R);
-      // one atomic instruction per run: lane k adds moment k of the run's
-      // cell, so the instruction's seven lanes hit one cache line (seven
-      // instructions with one lane per run each measured 2.3 ms more per
-      // full-form step: the L2 takes same-line lanes of an instruction
-      // together)
-      unsigned long long tails = __ballot(R.tail && live);
-      while (tails) {
-        const int t = __ffsll((long long)tails) - 1;
-        tails &= tails - 1ull;
-        const uint32_t kt = (uint32_t)__builtin_amdgcn_readlane((int)key, t);
-        float mine = 0.f;
-#pragma unroll
-        for (int k = 0; k < 7; ++k) {
-          const float qk = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(q[k]), t));
-          if (lane == k) mine = qk;
+        for (int k = 0; k < 7; ++k) q[k] = run_sum_f(q[k], R);
+      }
+      const bool tail = R.tail && live;
+      const unsigned long long tails = __ballot(tail);
+      const int runs = __popcll(tails), rank = __popcll(tails & ((1ull << lane) - 1ull));
+      for (int r0 = 0; r0 < runs; r0 += 8) {
+        if (tail && rank >= r0 && rank < r0 + 8) {
+          float4 *row = (float4 *)run[rank - r0];
+          row[0] = make_float4(q[0], q[1], q[2], q[3]);
+          row[1] = make_float4(q[4], q[5], q[6], __uint_as_float(key));
         }
-        if (lane < 7) atomicAdd(mom + (size_t)kt * SURR_PAR_STRIDE + slot * 8 + lane, (double)mine);
+        wave_lds_sync();
+        const int r = lane >> 3, k = lane & 7;
+        if (r0 + r < runs && k < 7) {
+          const uint32_t kt = __float_as_uint(run[r][7]);
+          atomicAdd(mom + (size_t)kt * SURR_PAR_STRIDE + slot * 8 + k, (double)run[r][k]);
+        }
+        wave_lds_sync();
       }
     }
   }
@@ -994,8 +1031,9 @@ __global__ void k32_gather_point(Geom g, FieldsT<float> f, int d, double r, doub
   float fr = (float)(ur - cr), fz = (float)(uz - cz);
   GridView32 V{(which == 0 ? f.E : f.H) + (long)d * 3 * g.P, g.P, g.yr, dm.bot_r, dm.left_z};
   float c[3];
-  if (which == 0) gather32_e(V, cr, cz, fr, fz, c);
-  else gather32_h(V, cr, cz, fr, fz, c);
+  const GatherWeights32 gw = gather_weights32(cr, cz, fr, fz);
+  if (which == 0) gather32_e(V, gw, c);
+  else gather32_h(V, gw, c);
   out[0] = c[0]; out[1] = c[1]; out[2] = c[2];
 }
 

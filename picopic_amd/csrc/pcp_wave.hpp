@@ -27,6 +27,14 @@ __device__ __forceinline__ double readlane64(double x, int lane) {
   return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
 }
 
+// LDS writes of the wavefront's lanes before, reads after (a wavefront's LDS
+// instructions stay in order; the compiler's must, too)
+__device__ __forceinline__ void wave_lds_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // Sum over the 64 lanes in a fixed order, returned to every lane: pairs and
 // quads by quad permutes, the 16-lane rows by row rotations (4 and 8), then
 // the four row sums.  All lanes must be active.
@@ -109,6 +117,51 @@ __device__ __forceinline__ float run_sum_f(float x, const Runs &R) {
   x = run_step_f<0x142>(x, R.m[4]);   // row_bcast:15
   x = run_step_f<0x143>(x, R.m[5]);   // row_bcast:31
   return x;
+}
+
+// run_sum_f of three or four values at once, a step being one multiply-add of
+// the shifted value with a mask of 1 or 0 (the product is exact, so the sum
+// rounds as run_sum_f's does; 6 instructions a value instead of 14 -- the FP32
+// particle kernels are bound by instruction issue and spent 15 to 30 % of it
+// on run sums).  A masked infinity would leave NaN in the next run: only for
+// values that run_sums_bounded accepts.  A DPP read needs two instructions
+// between it and the write of its register: the other values' steps.
+#define PCP_RUN_FMA(x, m, ctrl) "v_fmac_f32_dpp %" #x ", %" #x ", %" #m " " ctrl " bank_mask:0xf bound_ctrl:0\n\t"
+#define PCP_RUN_FMA3(m, ctrl) PCP_RUN_FMA(0, m, ctrl) PCP_RUN_FMA(1, m, ctrl) PCP_RUN_FMA(2, m, ctrl)
+#define PCP_RUN_FMA4(m, ctrl) PCP_RUN_FMA3(m, ctrl) PCP_RUN_FMA(3, m, ctrl)
+__device__ __forceinline__ float run_mask_f(const Runs &R, int s) { return __int_as_float(R.m[s] & 0x3f800000); }
+
+__device__ __forceinline__ void run_sums_f(float &a, float &b, float &c, const Runs &R) {
+  asm volatile("s_nop 1\n\t" PCP_RUN_FMA3(3, "row_shr:1 row_mask:0xf") PCP_RUN_FMA3(4, "row_shr:2 row_mask:0xf")
+                   PCP_RUN_FMA3(5, "row_shr:4 row_mask:0xf") PCP_RUN_FMA3(6, "row_shr:8 row_mask:0xf")
+                       PCP_RUN_FMA3(7, "row_bcast:15 row_mask:0xa")
+                           PCP_RUN_FMA3(8, "row_bcast:31 row_mask:0xc") "s_nop 1"
+               : "+v"(a), "+v"(b), "+v"(c)
+               : "v"(run_mask_f(R, 0)), "v"(run_mask_f(R, 1)), "v"(run_mask_f(R, 2)), "v"(run_mask_f(R, 3)),
+                 "v"(run_mask_f(R, 4)), "v"(run_mask_f(R, 5)));
+}
+
+__device__ __forceinline__ void run_sums_f(float &a, float &b, float &c, float &d, const Runs &R) {
+  asm volatile("s_nop 1\n\t" PCP_RUN_FMA4(4, "row_shr:1 row_mask:0xf") PCP_RUN_FMA4(5, "row_shr:2 row_mask:0xf")
+                   PCP_RUN_FMA4(6, "row_shr:4 row_mask:0xf") PCP_RUN_FMA4(7, "row_shr:8 row_mask:0xf")
+                       PCP_RUN_FMA4(8, "row_bcast:15 row_mask:0xa")
+                           PCP_RUN_FMA4(9, "row_bcast:31 row_mask:0xc") "s_nop 1"
+               : "+v"(a), "+v"(b), "+v"(c), "+v"(d)
+               : "v"(run_mask_f(R, 0)), "v"(run_mask_f(R, 1)), "v"(run_mask_f(R, 2)), "v"(run_mask_f(R, 3)),
+                 "v"(run_mask_f(R, 4)), "v"(run_mask_f(R, 5)));
+}
+#undef PCP_RUN_FMA
+#undef PCP_RUN_FMA3
+#undef PCP_RUN_FMA4
+
+// every lane's values are numbers, small enough that the sum of 64 of them is
+// finite (a NaN fails the comparison)
+template <int N>
+__device__ __forceinline__ bool run_sums_bounded(const float (&q)[N]) {
+  float s = fabsf(q[0]);
+#pragma unroll
+  for (int k = 1; k < N; ++k) s += fabsf(q[k]);
+  return __all(s < 0x1p120f);
 }
 
 // Compensated summation in FP32.  two_sum returns fl(a + b) and sets e to
