@@ -945,8 +945,12 @@ __global__ void k32_sort_tail(Species32 s, const uint32_t *n_live_ptr) {
   }
 }
 
-__global__ void k32_zero_u32(uint32_t *p, long n) {
-  for (long t = (long)blockIdx.x * blockDim.x + threadIdx.x; t < n; t += (long)gridDim.x * blockDim.x) p[t] = 0;
+// clears the sort's two counter arrays
+__global__ void k32_zero_u32(uint32_t *count, uint32_t *fill, long n) {
+  for (long t = (long)blockIdx.x * blockDim.x + threadIdx.x; t < n; t += (long)gridDim.x * blockDim.x) {
+    count[t] = 0;
+    fill[t] = 0;
+  }
 }
 
 __global__ void k32_count_live(const uint32_t *cell, long n, unsigned long long *out) {
@@ -1380,8 +1384,7 @@ int launch32_sort(pcp_ctx *c, int sp) {
   unsigned grid = pgrid32(c, s.n, 256);
   const unsigned gsort = (unsigned)std::max(1L, std::min((s.n + SORT_CHUNK - 1) / SORT_CHUNK, (long)c->n_cu * 16));
   unsigned gz = (unsigned)std::min<long>((ncells + 256) / 256, (long)c->n_cu * 16);
-  hipLaunchKernelGGL(k32_zero_u32, dim3(gz), dim3(256), 0, c->stream, c->sort_count, ncells + 1);
-  hipLaunchKernelGGL(k32_zero_u32, dim3(gz), dim3(256), 0, c->stream, c->sort_fill, ncells + 1);
+  hipLaunchKernelGGL(k32_zero_u32, dim3(gz), dim3(256), 0, c->stream, c->sort_count, c->sort_fill, ncells + 1);
   hipLaunchKernelGGL(k32_sort_count, dim3(gsort), dim3(SORT_BLOCK), 0, c->stream, c->g, s, c->cur, c->sort_key, c->sort_count,
                      sentinel);
   size_t bytes = c->sort_temp_bytes;

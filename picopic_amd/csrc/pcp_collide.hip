@@ -110,7 +110,8 @@ __device__ __forceinline__ uint32_t bucket_of(const Geom &g, const V &v, long p,
   return k;
 }
 
-// pass 1: particles per bucket (one atomic per distinct key of a wavefront)
+// pass 1: particles per bucket (one atomic per run of a bucket's particles in a
+// wavefront)
 template <class V>
 __global__ void __launch_bounds__(256) k_coll_count(Geom g, V v, uint32_t *cnt, uint32_t sentinel, const int *mask,
                                                     const unsigned long long *gate) {
@@ -121,7 +122,7 @@ __global__ void __launch_bounds__(256) k_coll_count(Geom g, V v, uint32_t *cnt, 
     const long p = b0 + threadIdx.x;
     const uint32_t k = bucket_of(g, v, p, n, sentinel, mask);
     const bool a = k != sentinel;
-    (void)wave_reserve(cnt, a ? k : 0, a);
+    (void)run_reserve(cnt, k, a);
   }
 }
 
@@ -139,7 +140,7 @@ __global__ void __launch_bounds__(256) k_coll_fill(Geom g, V v, const uint32_t *
     const long p = b0 + threadIdx.x;
     const uint32_t k = bucket_of(g, v, p, n, sentinel, mask);
     const bool a = k != sentinel;
-    const uint32_t slot = wave_reserve(fill, a ? k : 0, a);
+    const uint32_t slot = run_reserve(fill, k, a);
     if (a) perm[off[k] + slot] = (uint32_t)p;
   }
 }

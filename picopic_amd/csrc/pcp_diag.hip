@@ -333,26 +333,13 @@ __global__ void __launch_bounds__(256) k_map_heads(Geom g, V parts, long n, uint
   if (threadIdx.x == 0 && (c = part[0] + part[1] + part[2] + part[3])) atomicAdd(heads, c);
 }
 
-// slots of the lanes' keys counted up in ctr, one atomic per run of equal keys
-// in lane order; all 64 lanes call it
-__device__ __forceinline__ uint32_t run_reserve(uint32_t *ctr, uint32_t key) {
-  const int lane = __lane_id();
-  const uint32_t prev = (uint32_t)__shfl_up((int)key, 1, 64);
-  const unsigned long long heads = __ballot(lane == 0 || prev != key);
-  const int head = 63 - __clzll((long long)(heads & (~0ull >> (63 - lane))));
-  const unsigned long long after = lane == 63 ? 0ull : heads & (~0ull << (lane + 1));
-  const int next = after ? __ffsll((long long)after) - 1 : 64;
-  uint32_t base = 0;
-  if (lane == head && key != NO_CELL) base = atomicAdd(ctr + key, (uint32_t)(next - head));
-  return (uint32_t)__shfl((int)base, head, 64) + (uint32_t)(lane - head);
-}
-
 template <class V>
 __global__ void __launch_bounds__(256) k_map_count(Geom g, V parts, long n, const uint32_t *heads, uint32_t *cnt) {
   if (map_in_order(heads, n)) return;
   for (long b = (long)blockIdx.x * blockDim.x; b < n; b += (long)gridDim.x * blockDim.x) {
     const long p = b + threadIdx.x;
-    (void)run_reserve(cnt, p < n ? parts.cell(g, p) : NO_CELL);
+    const uint32_t c = p < n ? parts.cell(g, p) : NO_CELL;
+    (void)run_reserve(cnt, c, c != NO_CELL);
   }
 }
 
@@ -363,7 +350,7 @@ __global__ void __launch_bounds__(256) k_map_fill(Geom g, V parts, long n, const
   for (long b = (long)blockIdx.x * blockDim.x; b < n; b += (long)gridDim.x * blockDim.x) {
     const long p = b + threadIdx.x;
     const uint32_t c = p < n ? parts.cell(g, p) : NO_CELL;
-    const uint32_t slot = run_reserve(fill, c);
+    const uint32_t slot = run_reserve(fill, c, c != NO_CELL);
     if (c != NO_CELL) perm[off[c] + slot] = (uint32_t)p;
   }
 }
@@ -479,8 +466,12 @@ __global__ void k_map_derive(Geom g, int kind, double mass, const double *N, con
   }
 }
 
-__global__ void k_zero_u32(uint32_t *p, long n) {
-  for (long t = (long)blockIdx.x * blockDim.x + threadIdx.x; t < n; t += (long)gridDim.x * blockDim.x) p[t] = 0;
+// clears the sort's two counter arrays
+__global__ void k_zero_u32(uint32_t *count, uint32_t *fill, long n) {
+  for (long t = (long)blockIdx.x * blockDim.x + threadIdx.x; t < n; t += (long)gridDim.x * blockDim.x) {
+    count[t] = 0;
+    fill[t] = 0;
+  }
 }
 
 __global__ void k_zero_f64(double *p, long n) {
@@ -499,8 +490,7 @@ static int map_deposit(pcp_ctx *c, V parts, long n, double mass, int kind, doubl
   const unsigned gp = (unsigned)std::max(1L, std::min((n + 255) / 256, (long)c->n_cu * 16));
   // the last of the fill counters (one more than the cells) counts the order's breaks
   uint32_t *heads = c->sort_fill + ncells;
-  hipLaunchKernelGGL(k_zero_u32, dim3(gz), dim3(256), 0, c->stream, c->sort_fill, ncells + 1);
-  hipLaunchKernelGGL(k_zero_u32, dim3(gz), dim3(256), 0, c->stream, c->sort_count, ncells + 1);
+  hipLaunchKernelGGL(k_zero_u32, dim3(gz), dim3(256), 0, c->stream, c->sort_count, c->sort_fill, ncells + 1);
   // few workgroups: each ends with an atomic on the one counter
   const unsigned gh = std::min(gp, (unsigned)c->n_cu * 4);
   hipLaunchKernelGGL(k_map_heads<V>, dim3(gh), dim3(256), 0, c->stream, g, parts, n, heads);

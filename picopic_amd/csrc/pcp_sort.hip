@@ -63,8 +63,12 @@ __global__ void k_sort_tail(SpeciesDev s, const uint32_t *n_live_ptr) {
   }
 }
 
-__global__ void k_zero_u32(uint32_t *p, long n) {
-  for (long t = (long)blockIdx.x * blockDim.x + threadIdx.x; t < n; t += (long)gridDim.x * blockDim.x) p[t] = 0;
+// clears the sort's two counter arrays
+__global__ void k_zero_u32(uint32_t *count, uint32_t *fill, long n) {
+  for (long t = (long)blockIdx.x * blockDim.x + threadIdx.x; t < n; t += (long)gridDim.x * blockDim.x) {
+    count[t] = 0;
+    fill[t] = 0;
+  }
 }
 
 size_t sort_temp_bytes(long ncells) {
@@ -82,8 +86,7 @@ int launch_sort(pcp_ctx *c, int sp) {
   unsigned grid = (unsigned)std::min<long>((s.n + 255) / 256, (long)c->n_cu * 16);
   const unsigned gsort = (unsigned)std::max(1L, std::min((s.n + SORT_CHUNK - 1) / SORT_CHUNK, (long)c->n_cu * 16));
   unsigned gz = (unsigned)std::min<long>((ncells + 256) / 256, (long)c->n_cu * 16);
-  hipLaunchKernelGGL(k_zero_u32, dim3(gz), dim3(256), 0, c->stream, c->sort_count, ncells + 1);
-  hipLaunchKernelGGL(k_zero_u32, dim3(gz), dim3(256), 0, c->stream, c->sort_fill, ncells + 1);
+  hipLaunchKernelGGL(k_zero_u32, dim3(gz), dim3(256), 0, c->stream, c->sort_count, c->sort_fill, ncells + 1);
   hipLaunchKernelGGL(k_sort_count, dim3(gsort), dim3(SORT_BLOCK), 0, c->stream, c->g, s, c->cur, c->sort_key, c->sort_count,
                      sentinel);
   size_t bytes = c->sort_temp_bytes;
