@@ -4,7 +4,8 @@ hipcc compiles every ``csrc/*.hip`` into ``_lib/libpicopic_hip.so``.  FP64
 kernels are compiled without FMA contraction so their rounding follows the
 reference's IEEE build; packed FP32 instructions are disabled.  g++ then
 builds ``_lib/smb_driver``, an SMB-style C++ time loop over the drop-in
-solver objects of ``include/picopic_solvers.hpp``.
+solver objects of ``include/picopic_solvers.hpp``.  ``csrc/unit`` becomes
+``_lib/libpicopic_unit.so``, the helpers that the unit tests call directly.
 """
 import os
 import subprocess
@@ -14,7 +15,9 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 OUT_DIR = os.path.join(HERE, "_lib")
 LIB = os.path.join(OUT_DIR, "libpicopic_hip.so")
+UNIT = os.path.join(OUT_DIR, "libpicopic_unit.so")
 DRIVER = os.path.join(OUT_DIR, "smb_driver")
+UNIT_SRC = os.path.join(CSRC, "unit", "pcp_unit.hip")
 INCLUDE = os.path.join(os.path.dirname(HERE), "include")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = os.environ.get("PCP_OFFLOAD_ARCH", "gfx950")
@@ -47,7 +50,7 @@ def build(verbose=False):
     os.makedirs(OUT_DIR, exist_ok=True)
     objs = []
     jobs = []
-    for src in sources():
+    for src in sources() + [UNIT_SRC]:
         obj = os.path.join(OUT_DIR, os.path.basename(src)[:-4] + ".o")
         cmd = [HIPCC] + FLAGS + FILE_FLAGS.get(os.path.basename(src), []) + ["-c", src, "-o", obj]
         jobs.append((cmd, subprocess.Popen(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT)))
@@ -65,9 +68,10 @@ def build(verbose=False):
             sys.stderr.write("\n".join(lines) + "\n")
     if failed:
         raise RuntimeError("hipcc failed")
-    tmp = LIB + ".tmp"
-    subprocess.run([HIPCC, "--offload-arch=" + ARCH, "-shared", "-fPIC", "-o", tmp] + objs, check=True)
-    os.replace(tmp, LIB)
+    for lib, parts in ((LIB, objs[:-1]), (UNIT, objs[-1:])):
+        tmp = lib + ".tmp"
+        subprocess.run([HIPCC, "--offload-arch=" + ARCH, "-shared", "-fPIC", "-o", tmp] + parts, check=True)
+        os.replace(tmp, lib)
     for o in objs:
         os.remove(o)
     build_driver()

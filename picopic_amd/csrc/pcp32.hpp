@@ -47,32 +47,36 @@ struct SortBuffers32 {
 };
 
 // Cell and FP32 in-cell offset of a coordinate u (cell units) of a grid of n
-// cells.  An offset that rounds to 1 moves to the next cell -- at the last cell
-// it stays at the largest offset below 1: the cell past it is outside the grid.
-__host__ __device__ __forceinline__ void split_coordinate(double u, long n, long &cell, float &f) {
+// cells; false, and nothing written, where u lies outside the grid (or is no
+// number).  An offset that rounds to 1 moves to the next cell -- in the last
+// cell it stays at the largest offset below 1: the cell past it is outside.
+__host__ __device__ __forceinline__ bool split_coordinate(double u, long n, long &cell, float &f) {
   const double fc = floor(u);
+  if (!(fc >= 0 && fc < (double)n)) return false;
   cell = (long)fc;
   f = (float)(u - fc);
   if (f >= 1.f) {
-    f = 0.f;
-    cell += 1;
+    if (cell == n - 1) {
+      f = 1.f - 0x1p-24f;
+    } else {
+      f = 0.f;
+      cell += 1;
+    }
   }
-  if (cell >= n) {
-    cell = n - 1;
-    f = 1.f - 0x1p-24f;
-  }
+  return true;
 }
 
-// position (r, z) in split form, written to both position slots of q
-__device__ __forceinline__ void store_split(Species32 &s, long q, const Geom &g, double r, double z) {
-  long cr, cz;
-  float fr, fz;
-  split_coordinate(r / g.dr, g.Nr, cr, fr);
-  split_coordinate(z / g.dz, g.Nz, cz, fz);
-  uint32_t cell = (uint32_t)cr * (uint32_t)g.Nz + (uint32_t)cz;
+// position (r, z) in split form, written to both position slots of q; outside
+// the grid (false) q becomes a removed particle
+__device__ __forceinline__ bool store_split(Species32 &s, long q, const Geom &g, double r, double z) {
+  long cr = 0, cz = 0;
+  float fr = 0.f, fz = 0.f;
+  const bool in_r = split_coordinate(r / g.dr, g.Nr, cr, fr), in_z = split_coordinate(z / g.dz, g.Nz, cz, fz);
+  uint32_t cell = in_r && in_z ? (uint32_t)cr * (uint32_t)g.Nz + (uint32_t)cz : DEAD_CELL;
   s.cell[0][q] = cell; s.cell[1][q] = cell;
   s.fr[0][q] = fr; s.fr[1][q] = fr;
   s.fz[0][q] = fz; s.fz[1][q] = fz;
+  return in_r && in_z;
 }
 
 // state of an FP32 context (owned by pcp_ctx)

@@ -438,9 +438,9 @@ int pcp_upload_species(pcp_ctx *c, int sp, long n, const double *r, const double
     std::vector<uint32_t> cell(n);
     std::vector<float> fr(n), fz(n), fvr(n), fvp(n), fvz(n), fw(n);
     for (long p = 0; p < n; ++p) {
-      long ir, iz;
-      split_coordinate(r[p] / g.dr, g.Nr, ir, fr[p]);
-      split_coordinate(z[p] / g.dz, g.Nz, iz, fz[p]);
+      long ir = 0, iz = 0;   // inside the grid, as checked above
+      (void)split_coordinate(r[p] / g.dr, g.Nr, ir, fr[p]);
+      (void)split_coordinate(z[p] / g.dz, g.Nz, iz, fz[p]);
       cell[p] = (uint32_t)(ir * g.Nz + iz);
       fvr[p] = (float)vr[p]; fvp[p] = (float)vphi[p]; fvz[p] = (float)vz[p]; fw[p] = (float)w[p];
     }
@@ -797,9 +797,10 @@ static long inject_beams(pcp_ctx *c) {
           const double v_macro_avg = PI * b.radius * dr * dz;
           const double N_total = PI * b.radius * b.radius * b.bunch_length * b.bunches_amount * b.density;
           const double n_per_macro_avg = N_total / b.macro_amount;
-          // particles past the domain's cells (a bunch wider than the domain)
-          const bool spill = B.domain_radius + dr / 2 + dm.bot_r * dr >= (dm.bot_r + g.nr) * dr ||
-                             dl + dz / 2. >= g.nz * dz;
+          // particles past the domain's cells (a bunch wider than the domain;
+          // an FP32 offset rounds into the next cell 2^-25 of a cell before it)
+          const bool spill = B.domain_radius + dr / 2 + dm.bot_r * dr >= (dm.bot_r + g.nr - 1e-6) * dr ||
+                             dl + dz / 2. >= (g.nz - 1e-6) * dz;
           launch_inject(c, sp, c->sp[sp].n, n, d, B.domain_radius, dl, b.velocity, v_macro_avg, n_per_macro_avg,
                         b.seed, B.injected, spill);
           if (spill) {

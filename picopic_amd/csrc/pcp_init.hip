@@ -82,12 +82,29 @@ __global__ void k_init_bunch(Geom g, SpeciesDev s, long base, long n_new, double
   }
 }
 
+// domain of position (r, z); false outside the grid (or no number)
+__device__ __forceinline__ bool grid_owner(const Geom &g, double r, double z, int &d) {
+  const int cr = cell_number(r, g.dr), cz = cell_number(z, g.dz);
+  if (!(r >= 0 && z >= 0) || cr >= g.Nr || cz >= g.Nz) return false;
+  d = domain_of(g, cr, cz);
+  return true;
+}
+// the same of the stored split position of particle q
+__device__ __forceinline__ bool split_owner(Species32 &s, long q, const Geom &g, double r, double z, int &d) {
+  if (!store_split(s, q, g, r, z)) return false;
+  const uint32_t cell = s.cell[0][q];
+  const int cr = (int)g.div_Nz.div(cell);
+  d = domain_of(g, cr, (int)(cell - (uint32_t)cr * (uint32_t)g.Nz));
+  return true;
+}
+
 // The reference's initial distribution of one plasma species: particle
 // k of domain d (M per domain) goes to slot base + d M + k.  A particle that
 // the domain places beyond its own cells (inner domain edges are not walls,
 // src/specieP.cpp:148-149) is a migrant of the first runaway collector: it
 // is appended to the migrant list with its generating domain's key and
-// takes its order key in the owning domain from the migration pass.
+// takes its order key in the owning domain from the migration pass.  One
+// that rounding places outside the grid is removed, as that collector does.
 template <bool F32>
 __global__ void k_init_reference(Geom g, SpeciesDev s64, Species32 s32, int sp, long base, uint32_t M,
                                  const RefInitDom *doms, RadicalPowers pw, double temperature, double mass,
@@ -102,8 +119,9 @@ __global__ void k_init_reference(Geom g, SpeciesDev s64, Species32 s32, int sp, 
     if (!ref_init_particle(g, P, pw, M, k, d, temperature, mass, seed, r, z, v, w)) err |= ERR_NAN_POSITION;
     const long q = base + p;
     const uint64_t seq = P.seq_base + k;
+    int d_own;
+    const bool inside = F32 ? split_owner(s32, q, g, r, z, d_own) : grid_owner(g, r, z, d_own);
     if (F32) {
-      store_split(s32, q, g, r, z);
       s32.vr[0][q] = s32.vr[1][q] = (float)v[0];
       s32.vphi[0][q] = s32.vphi[1][q] = (float)v[1];
       s32.vz[0][q] = s32.vz[1][q] = (float)v[2];
@@ -111,7 +129,7 @@ __global__ void k_init_reference(Geom g, SpeciesDev s64, Species32 s32, int sp, 
       s32.seq[q] = seq;
       s32.id[q] = (uint64_t)q;
     } else {
-      s64.r[0][q] = r; s64.r[1][q] = r;
+      s64.r[0][q] = s64.r[1][q] = inside ? r : -1;
       s64.z[0][q] = z; s64.z[1][q] = z;
       s64.vr[q] = v[0];
       s64.vphi[q] = v[1];
@@ -120,15 +138,7 @@ __global__ void k_init_reference(Geom g, SpeciesDev s64, Species32 s32, int sp, 
       s64.seq[q] = seq;
       s64.id[q] = (uint64_t)q;
     }
-    int d_own;
-    if (F32) {
-      const uint32_t cell = s32.cell[0][q];
-      const int cr = (int)g.div_Nz.div(cell);
-      d_own = domain_of(g, cr, (int)(cell - (uint32_t)cr * (uint32_t)g.Nz));
-    } else {
-      d_own = domain_of(g, cell_number(r, g.dr), cell_number(z, g.dz));
-    }
-    if (d_own != d) append_migrant(mg, st, sp, q, d, d_own, seq, g, &err);
+    if (inside && d_own != d) append_migrant(mg, st, sp, q, d, d_own, seq, g, &err);
   }
   if (err) atomicOr(&st->err, err);
 }
@@ -139,7 +149,9 @@ __global__ void k_reset_migrants(StepState *st) { st->n_mig = 0; }
 // reference's two uniforms per particle are Philox draw 0 of counter
 // (d << 40 | ctr0 + i); the particles take order keys after every particle
 // of (d, sp) (appended to the domain's vector); one placed past the domain's
-// cells is a migrant to its owner.
+// cells is a migrant to its owner, one past the grid (a beam's radius may
+// reach half a cell beyond the wall) is removed, as the runaway collector
+// does.
 template <bool F32>
 __global__ void k_inject(Geom g, SpeciesDev s64, Species32 s32, int sp, long base, long n, int d, double domain_radius,
                          double dl, double velocity, double v_macro_avg, double n_per_macro_avg, uint64_t seed,
@@ -163,8 +175,9 @@ __global__ void k_inject(Geom g, SpeciesDev s64, Species32 s32, int sp, long bas
     const long q = base + i;
     const uint64_t seq = seq_base + (uint64_t)i;
     const uint64_t id = (1ull << 62) | ctr;
+    int d_own;
+    const bool inside = F32 ? split_owner(s32, q, g, pos_r, pos_z, d_own) : grid_owner(g, pos_r, pos_z, d_own);
     if (F32) {
-      store_split(s32, q, g, pos_r, pos_z);
       s32.vr[0][q] = s32.vr[1][q] = 0.f;
       s32.vphi[0][q] = s32.vphi[1][q] = 0.f;
       s32.vz[0][q] = s32.vz[1][q] = (float)velocity;
@@ -172,7 +185,7 @@ __global__ void k_inject(Geom g, SpeciesDev s64, Species32 s32, int sp, long bas
       s32.seq[q] = seq;
       s32.id[q] = id;
     } else {
-      s64.r[0][q] = pos_r; s64.r[1][q] = pos_r;
+      s64.r[0][q] = s64.r[1][q] = inside ? pos_r : -1;
       s64.z[0][q] = pos_z; s64.z[1][q] = pos_z;
       s64.vr[q] = 0;
       s64.vphi[q] = 0;
@@ -181,15 +194,7 @@ __global__ void k_inject(Geom g, SpeciesDev s64, Species32 s32, int sp, long bas
       s64.seq[q] = seq;
       s64.id[q] = id;
     }
-    int d_own;
-    if (F32) {
-      const uint32_t cell = s32.cell[0][q];
-      const int cr = (int)g.div_Nz.div(cell);
-      d_own = domain_of(g, cr, (int)(cell - (uint32_t)cr * (uint32_t)g.Nz));
-    } else {
-      d_own = domain_of(g, cell_number(pos_r, dr), cell_number(pos_z, dz));
-    }
-    if (d_own != d) append_migrant(mg, st, sp, q, d, d_own, seq, g, &err);
+    if (inside && d_own != d) append_migrant(mg, st, sp, q, d, d_own, seq, g, &err);
   }
   if (err) atomicOr(&st->err, err);
 }

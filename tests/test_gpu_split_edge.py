@@ -1,12 +1,14 @@
-"""FP32 split positions next to the outer edges of the grid.
+"""Positions next to the outer edges of the grid and past them.
 
-A coordinate within 2^-25 of a cell below the grid's end has an in-cell offset
-that rounds to 1, which must not carry it into the cell past the last one (the
-sort's counters and the field grids end there).
+A coordinate within 2^-25 of a cell below the grid's end has an FP32 in-cell
+offset that rounds to 1, which must not carry it into the cell past the last
+one (the sort's counters and the field grids end there).  A beam's particles
+placed past the grid are removed.
 """
 import numpy as np
 import pytest
 
+from oracle import oracle as O
 from picopic_amd import capi
 
 pytestmark = pytest.mark.gpu
@@ -43,3 +45,31 @@ def test_initial_plasma_stays_in_the_last_cell():
     print("init_plasma", flush=True)
     p = check(ctx, grid)
     assert len(p["r"]) == 80000 and p["r"].max() > (2 - 1e-6) * CELL
+
+
+@pytest.mark.parametrize("radius", [0.9, 1.0, 1.25])
+@pytest.mark.parametrize("domains", [(1, 1), (2, 2)])
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+def test_beam_as_wide_as_the_grid(precision, domains, radius):
+    """A beam's particles reach half a cell past its radius: the ones outside the grid are removed, as the oracle's
+    runaway collector does, and the rest are the oracle's, before and after steps."""
+    size, grid, dt = (8.0, 8.0), (8, 8), 1.0
+    species = [(-1, 1, False), (-1, 1, True)]
+    orc = O.SMB(size, grid, domains, dt, species)
+    dev = capi.Context(size, grid, domains, dt, [s + (4096,) for s in species], precision=precision)
+    print("wide beam", precision, domains, radius, flush=True)
+    for s in (orc, dev):
+        s.set_beam(1, 900, 0.0, radius * size[0], 1e-12, 1, 3.0, 2.0, 1.0, seed=5)
+        for _ in range(3):
+            s.inject()
+            s.set_time(s.time() + dt)
+    a, b = orc.particles(1), dev.particles(1)
+    ia, ib = np.argsort(a["id"]), np.argsort(b["id"])
+    assert len(ia) > 500 and np.array_equal(a["id"][ia], b["id"][ib])
+    for k in ("r", "z", "vz", "w"):
+        tol = 0 if precision == "fp64" else 1e-6
+        assert np.abs(a[k][ia] - b[k][ib]).max() <= tol * np.abs(a[k]).max(), k
+    assert b["r"].max() < size[0]
+    for s in (orc, dev):
+        s.step(2)
+    assert orc.count(1) == dev.count(1)
