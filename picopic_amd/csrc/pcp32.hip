@@ -988,8 +988,8 @@ __global__ void k32_init_plasma(Geom g, Species32 s, long base, long n_new, cons
     double r = sqrt(r0 * r0 + u0 * (r1 * r1 - r0 * r0));
     double z = (gk + u1) * g.dz;
     if (r < r0) r = r0;
-    if (r >= r1) r = nextafter(r1, 0.0);
-    if (z >= (gk + 1) * g.dz) z = nextafter((gk + 1) * g.dz, 0.0);
+    r = fmin(r, below_edge(gi, g.dr));
+    z = fmin(z, below_edge(gk, g.dz));
     long q = base + p;
     store_split(s, q, g, r, z);
     s.vr[0][q] = s.vr[1][q] = (float)(n0 * vth);

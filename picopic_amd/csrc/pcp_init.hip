@@ -40,8 +40,8 @@ __global__ void k_init_plasma(Geom g, SpeciesDev s, long base, long n_new, const
     double z = (gk + u1) * g.dz;
     // keep the particle inside its cell
     if (r < r0) r = r0;
-    if (r >= r1) r = nextafter(r1, 0.0);
-    if (z >= (gk + 1) * g.dz) z = nextafter((gk + 1) * g.dz, 0.0);
+    r = fmin(r, below_edge(gi, g.dr));
+    z = fmin(z, below_edge(gk, g.dz));
     long q = base + p;
     s.r[0][q] = r; s.r[1][q] = r;
     s.z[0][q] = z; s.z[1][q] = z;

@@ -181,6 +181,15 @@ __host__ __device__ inline double *ehist_row(double *h, unsigned long long step)
   return h + (long)(step % EHIST) * EHIST_COLS;
 }
 
+// The upper limit of a coordinate placed in cell i of cells dx wide.  The
+// neighbour of (i + 1) dx below it is not one: its quotient by dx can round to
+// i + 1 (i + 1 = 9 and dx = 1e-3, for instance), in the last cell an index
+// past the grid.  Four units further down it lies below i + 1 however product
+// and quotient round.
+__host__ __device__ __forceinline__ double below_edge(long i, double dx) {
+  return (double)(i + 1) * dx * (1.0 - 0x1p-50);
+}
+
 // domain owning global cell (cr, cz) (a cell below the grid, which a particle
 // that is not collected yet can be in, divides toward zero)
 __device__ __forceinline__ int domain_of(const Geom &g, int cr, int cz) {

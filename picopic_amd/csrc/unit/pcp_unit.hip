@@ -15,6 +15,11 @@ void unit_split(long n, const double *u, long nc, int *inside, long *cell, float
   for (long k = 0; k < n; ++k) inside[k] = split_coordinate(u[k], nc, cell[k], f[k]) ? 1 : 0;
 }
 
+// below_edge of the cells i[k]
+void unit_below_edge(long n, const long *i, double dx, double *x) {
+  for (long k = 0; k < n; ++k) x[k] = below_edge(i[k], dx);
+}
+
 // sort keys of the global cells (cr[k], cz[k]) of a grid of Dr x Dz domains of
 // nr x nz cells in bins of bin_r x bin_z
 void unit_sort_keys(long n, const long *cr, const long *cz, int Dr, int Dz, int nr, int nz, int bin_r, int bin_z,

@@ -49,6 +49,19 @@ def test_the_ion_that_left_the_grid():
     assert inside[0] and cell[0] == 1023 and f[0] < 1
 
 
+@pytest.mark.parametrize("dx", [1e-3, 1e-6, 0.0375 / 128, 0.15 / 256, 1.1e-3, 0.7])
+def test_the_upper_limit_of_a_cell_is_in_it(dx):
+    i = np.arange(9000, dtype=np.int64)
+    x = np.zeros(len(i))
+    U.unit_below_edge(C.c_long(len(i)), ptr(i), C.c_double(dx), ptr(x))
+    for q in (x / dx, x * (1 / dx)):
+        assert np.array_equal(np.floor(q), i)
+    assert np.abs(x / dx - (i + 1)).max() <= 9000 * 2.0 ** -49
+    # the neighbour below the edge is not such a limit everywhere
+    if dx == 1e-3:
+        assert (np.floor(np.nextafter((i + 1) * dx, 0.0) / dx) > i).any()
+
+
 @pytest.mark.parametrize("dr,dz,nr,nz,bin_r,bin_z", [(1, 1, 8, 16, 1, 16), (8, 8, 128, 512, 16, 32), (8, 2, 128, 512, 16, 32),
                                                     (2, 4, 64, 64, 16, 32), (1, 1, 125, 511, 5, 7), (3, 2, 5, 9, 1, 3)])
 def test_sort_keys_count_every_cell_once(dr, dz, nr, nz, bin_r, bin_z):
