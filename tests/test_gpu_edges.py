@@ -75,3 +75,19 @@ def test_empty_and_ragged_species(precision, ccs, domains, counts):
         e = Hh.relerr(gpu.get_grid(nm)[:, :, 2:-2, 2:-2], orc.get_grid(nm)[:, :, 2:-2, 2:-2])
         print(nm, e)
         assert e <= tol_f, (nm, e)
+
+
+@pytest.mark.parametrize("speed", [3.1e8, 1e200, np.inf])
+@pytest.mark.parametrize("pusher", ["boris-adaptive", "vay", "hc"])
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+def test_faster_than_light_is_an_error(precision, pusher, speed):
+    """Also where v^2 / c^2 overflows: the step reports it rather than dropping the particle in silence."""
+    from picopic_amd import capi
+    ctx = capi.Context((8e-3, 8e-3), (8, 8), (1, 1), 1e-13, [(-1, 1, False, 64)], pusher=pusher, precision=precision)
+    x, zero = np.full(3, 4.2e-3), np.zeros(3)
+    print("beta", precision, pusher, speed, flush=True)
+    with np.errstate(over="ignore"):
+        ctx.upload(0, x, x, zero, zero, np.array([1e6, speed, 2e6]), zero + 1e6)
+        with pytest.raises(capi.PcpError, match="0x2|0x3"):
+            ctx.step(1)
+            ctx.sync()
