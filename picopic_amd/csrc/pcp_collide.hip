@@ -34,6 +34,7 @@
 #include "pcp_collide.hpp"
 #include "pcp_collide_physics.hpp"
 #include "pcp_mlp.hpp"
+#include "pcp_pair_schedule.hpp"
 #include "pcp_rng.hpp"
 #include "pcp_wave.hpp"
 
@@ -509,19 +510,6 @@ struct CrowdStage {
   __device__ __forceinline__ double &w(int s, int k) const { return at(3, s, k); }
 };
 
-__device__ __forceinline__ uint32_t like_pairs(int n) {
-  if (n % 2 == 0) return (uint32_t)(n / 2);
-  return (uint32_t)((n >= 3 ? 3 : 0) + (n >= 5 ? (n - 3) / 2 : 0));
-}
-
-// the threads that run a crowded cell's loops split the independent pairs of
-// a phase
-struct BlockTeam {
-  static constexpr int step = COLL_CROWD_BLOCK;
-  __device__ __forceinline__ int first() const { return (int)threadIdx.x; }
-  __device__ __forceinline__ void sync() const { __syncthreads(); }
-};
-
 // One pair, out of line: the schedule below calls it from several places.  Only
 // the arithmetic is: with the draws and the stage's loads inside the call the
 // runner's state went through scratch (SK98 146 -> 244 registers).  The serial
@@ -537,11 +525,11 @@ __device__ __noinline__ void collide_pair_call(double m_a, double m_b, double q_
   collide_pair<SCHEME>(m_a, m_b, q_a, q_b, va, wa, vb, wb, dens_a, dens_b, K, debye, dt, R, err);
 }
 
-// the pair schedule of one cell (collisionsP12.cpp:356-528)
-template <int SCHEME, class Stage, class Team>
+// The pairs of a crowded cell, its independent pairs and chains spread over the
+// workgroup's threads
+template <int SCHEME>
 struct PairRunner {
-  Stage S;
-  Team T;
+  CrowdStage S;
   double m[2], q[2];   // electrons, ions
   double dens[2], debye, dt;
   uint64_t seed, step, gcell;
@@ -564,92 +552,39 @@ struct PairRunner {
   // like-particle pairs of species s (cases 1a / 1b), ordinals from qb
   __device__ void like(int s, int n, uint32_t qb) {
     if (n % 2 == 0) {
-      for (int k = T.first(); k < n / 2; k += Team::step) pair(s, 2 * k, s, 2 * k + 1, qb + (uint32_t)k);
+      for (int k = threadIdx.x; k < n / 2; k += COLL_CROWD_BLOCK) pair(s, 2 * k, s, 2 * k + 1, qb + (uint32_t)k);
     } else {
-      if (n >= 3 && T.first() == 0) {
+      if (n >= 3 && threadIdx.x == 0) {
         pair(s, 0, s, 1, qb);
         pair(s, 1, s, 2, qb + 1);
         pair(s, 2, s, 0, qb + 2);
       }
       if (n >= 5)
-        for (int k = T.first(); k < (n - 3) / 2; k += Team::step)
+        for (int k = threadIdx.x; k < (n - 3) / 2; k += COLL_CROWD_BLOCK)
           pair(s, 3 + 2 * k, s, 4 + 2 * k, qb + 3 + (uint32_t)k);
     }
+    __syncthreads();
+  }
+  __device__ void run(int nel, int nion) {
+    // cases 1a/1b in reference order: ion pairs if nion is even, electron pairs
+    // if nel is even, ion pairs if nion is odd, electron pairs if nel is odd
+    const uint32_t n_ion = like_pairs(nion), n_el = like_pairs(nel);
+    const bool el_first = nion % 2 != 0 && nel % 2 == 0;
+    like(1, nion, el_first ? n_el : 0);
+    like(0, nel, el_first ? 0 : n_ion);
+    // case 2a / 2b
+    UnlikeChains U;
+    U.set(nel, nion);
+    for (int e = threadIdx.x; e < U.n; e += COLL_CROWD_BLOCK) {
+      const int len = U.length(e);
+      for (int j = 0; j < len; ++j) {
+        const int far = U.partner(e, j);
+        pair(0, nel <= nion ? e : far, 1, nel <= nion ? far : e, n_ion + n_el + (uint32_t)far);
+      }
+    }
+    __syncthreads();
   }
 };
-
-__device__ __forceinline__ int grp(unsigned f, float div) { return (int)floorf((float)f / div); }
-
-// cases 1a/1b then 2a/2b of one cell
-template <class Runner>
-__device__ void cell_pairs(Runner &P, int nel, int nion) {
-  const auto &T = P.T;
-  constexpr int STEP = decltype(P.T)::step;
-  // cases 1a/1b in reference order: ions even, electrons even, ions odd, electrons odd
-  const uint32_t n_ion = like_pairs(nion), n_el = like_pairs(nel);
-  // blocks in reference order: ion pairs if nion is even, electron pairs
-  // if nel is even, ion pairs if nion is odd, electron pairs if nel is odd
-  uint32_t q_ion = 0, q_el = n_ion;
-  if (nion % 2 != 0 && nel % 2 == 0) { q_el = 0; q_ion = n_el; }
-  P.like(1, nion, q_ion);
-  T.sync();
-  P.like(0, nel, q_el);
-  T.sync();
-  const uint32_t qc = n_ion + n_el;
-  // case 2a / 2b
-  if (nion == nel) {
-    for (int k = T.first(); k < nel; k += STEP) P.pair(0, k, 1, k, qc + (uint32_t)k);
-  } else if (nion > nel && nel > 0) {
-    unsigned int c_i = (unsigned int)floorf((float)nion / (float)nel);
-    double c_r = (double)((float)nion / (float)nel - (float)c_i);
-    unsigned int ions_1st = (unsigned int)((c_i + 1) * c_r * nel);
-    unsigned int els_1st = (unsigned int)(c_r * nel);
-    unsigned int ions_2nd = (unsigned int)(c_i * (1 - c_r) * nel);
-    const float d1 = (float)(c_i + 1), d2 = (float)c_i;
-    // 1st group: electron e meets ions fgi with floor(fgi / (c_i + 1)) == e
-    for (int e = T.first(); e < nel; e += STEP) {
-      unsigned lo = (unsigned)e * (c_i + 1);
-      lo = lo > 0 ? lo - 1 : 0;
-      for (unsigned fgi = lo; fgi < ions_1st && fgi <= (unsigned)(e + 1) * (c_i + 1); ++fgi)
-        if (grp(fgi, d1) == e && (int)fgi < nion) P.pair(0, e, 1, (int)fgi, qc + fgi);
-    }
-    T.sync();
-    for (int e = T.first(); e < nel; e += STEP) {
-      if (e < (int)els_1st) continue;
-      int le = e - (int)els_1st;
-      unsigned lo = (unsigned)le * c_i;
-      lo = lo > 0 ? lo - 1 : 0;
-      for (unsigned fgi = lo; fgi < ions_2nd && fgi <= (unsigned)(le + 1) * c_i; ++fgi)
-        if (grp(fgi, d2) == le && (int)(fgi + ions_1st) < nion)
-          P.pair(0, e, 1, (int)(fgi + ions_1st), qc + ions_1st + fgi);
-    }
-  } else if (nion < nel && nion > 0) {
-    double c_i = floorf((float)nel / (float)nion);
-    double c_r = (double)((float)nel / (float)nion) - c_i;
-    unsigned int els_1st = (unsigned int)((c_i + 1) * c_r * nion);
-    unsigned int ions_1st = (unsigned int)(c_r * nion);
-    unsigned int els_2nd = (unsigned int)(c_i * (1 - c_r) * nion);
-    const float d1 = (float)(c_i + 1), d2 = (float)c_i;
-    const unsigned ci1 = (unsigned)c_i + 1, ci0 = (unsigned)c_i;
-    for (int i = T.first(); i < nion; i += STEP) {
-      unsigned lo = (unsigned)i * ci1;
-      lo = lo > 0 ? lo - 1 : 0;
-      for (unsigned fge = lo; fge < els_1st && fge <= (unsigned)(i + 1) * ci1; ++fge)
-        if (grp(fge, d1) == i && (int)fge < nel) P.pair(0, (int)fge, 1, i, qc + fge);
-    }
-    T.sync();
-    for (int i = T.first(); i < nion; i += STEP) {
-      if (i < (int)ions_1st) continue;
-      int li = i - (int)ions_1st;
-      unsigned lo = (unsigned)li * ci0;
-      lo = lo > 0 ? lo - 1 : 0;
-      for (unsigned fge = lo; fge < els_2nd && fge <= (unsigned)(li + 1) * ci0; ++fge)
-        if (grp(fge, d2) == li && (int)(fge + els_1st) < nel)
-          P.pair(0, (int)(fge + els_1st), 1, i, qc + els_1st + fge);
-    }
-  }
-  T.sync();
-}
 
 // TA77S correct_velocities for species s of the staged cell; t = the cell's
 // {amount, energy, moment[3]} from before the collisions
@@ -692,63 +627,22 @@ __device__ CorrParams correct_params(const Stage &S, int s, int n, double mass, 
   return P;
 }
 
-template <class Stage, class Team>
-__device__ void correct_species(const Stage &S, const Team &T, int s, int n, double mass, const double *t) {
+__device__ void correct_species(const CrowdStage &S, int s, int n, double mass, const double *t) {
   __shared__ CorrParams shared_p;
   if (threadIdx.x == 0) shared_p = correct_params(S, s, n, mass, t);
   __syncthreads();
   const CorrParams P = shared_p;
   if (P.ok != 0.0) {
     const double alpha = P.alpha;
-    for (int k = T.first(); k < n; k += Team::step) {
+    for (int k = threadIdx.x; k < n; k += COLL_CROWD_BLOCK) {
       double vr = S.vx(s, k), vphi = S.vy(s, k), vz = S.vz(s, k);
       S.vx(s, k) = P.V0[0] + alpha * (vr - P.V0[0] - P.dV[0]);
       S.vy(s, k) = P.V0[1] + alpha * (vphi - P.V0[1] - P.dV[1]);
       S.vz(s, k) = P.V0[2] + alpha * (vz - P.V0[2] - P.dV[2]);
     }
   }
-  T.sync();
+  __syncthreads();
 }
-
-// The unlike pairs of a cell with N particles of the more numerous species
-// and n of the other (cases 2a / 2b): each of the n meets a chain of the N,
-// first particles of the reference's 1st group (c + 1 each), then of the 2nd
-// (c each).  No particle of the N is in two chains, so the chains are
-// independent and each runs in the reference's order.
-struct UnlikeChains {
-  int n, big, c;                 // chains, N, floor(N / n)
-  int big1, small1, big2;        // 1st group: particles of the N, of the n; 2nd group: of the N
-  __device__ __forceinline__ void set(int nel, int nion) {
-    const int lo = min(nel, nion), hi = max(nel, nion);
-    n = lo;
-    big = hi;
-    if (lo == hi || lo == 0) {
-      c = 1;
-      big1 = small1 = 0;
-      big2 = lo;
-      return;
-    }
-    const float ratio = (float)hi / (float)lo;
-    const double ci = (double)floorf(ratio);
-    const double cr = (double)ratio - ci;
-    c = (int)ci;
-    big1 = min((int)((ci + 1) * cr * lo), hi);
-    small1 = (int)(cr * lo);
-    big2 = min((int)(ci * (1 - cr) * lo), hi - big1);
-  }
-  // chain e: pairs of the 1st and of both groups
-  __device__ __forceinline__ int first(int e) const { return min(max(big1 - e * (c + 1), 0), c + 1); }
-  __device__ __forceinline__ int length(int e) const {
-    return first(e) + (e >= small1 ? min(max(big2 - (e - small1) * c, 0), c) : 0);
-  }
-  // the N's particle (and pair ordinal) of pair j of chain e
-  __device__ __forceinline__ int partner(int e, int j) const {
-    const int f = first(e);
-    return j < f ? e * (c + 1) + j : big1 + (e - small1) * c + (j - f);
-  }
-  // chains that can hold more than one pair: every one for c > 1, else the 1st group's
-  __device__ __forceinline__ int long_chains() const { return c > 1 ? n : min(n, small1 + 1); }
-};
 
 // what a pair takes from its cell
 struct CellStatsLds {
@@ -1070,7 +964,6 @@ __global__ void __launch_bounds__(COLL_CROWD_BLOCK) k_coll_pairs_crowd(
   const uint64_t step = pass.get();
   if (gate_closed(gate)) return;
   const uint32_t nlist = *count;
-  const BlockTeam T;
   int err = 0;
   for (uint32_t li = blockIdx.x; li < nlist; li += gridDim.x) {
     const long c = list[li];
@@ -1082,15 +975,15 @@ __global__ void __launch_bounds__(COLL_CROWD_BLOCK) k_coll_pairs_crowd(
     const CellPos q = cell_pos(g, c);
     const double *t = tot + c * TOT;
     if (q.j < row_bad[(long)q.d * g.nr + q.i]) {
-      PairRunner<SCHEME, CrowdStage, BlockTeam> P{S, T, {m_e, m_i}, {q_e, q_i}, {t[10], t[11]}, t[12], g.dt, seed,
-                                                  step, (uint64_t)q.cr * (uint64_t)g.Nz + (uint64_t)q.cz, &err, {}};
+      PairRunner<SCHEME> P{S, {m_e, m_i}, {q_e, q_i}, {t[10], t[11]}, t[12], g.dt, seed, step,
+                           (uint64_t)q.cr * (uint64_t)g.Nz + (uint64_t)q.cz, &err, {}};
       if (SCHEME == COLL_P12)
         for (int k = 0; k < 3; ++k) P.K[k].set_species(k, m_e, m_i, q_e, q_i, t + 10, g.dt);
-      cell_pairs(P, nn[0], nn[1]);
+      P.run(nn[0], nn[1]);
     }
     if (SCHEME == COLL_TA77S) {
-      correct_species(S, T, 1, nn[1], m_i, t + 5);
-      correct_species(S, T, 0, nn[0], m_e, t + 0);
+      correct_species(S, 1, nn[1], m_i, t + 5);
+      correct_species(S, 0, nn[0], m_e, t + 0);
     }
     for (int k = threadIdx.x; k < nn[0]; k += COLL_CROWD_BLOCK) {
       double v3[3] = {S.vx(0, k), S.vy(0, k), S.vz(0, k)};

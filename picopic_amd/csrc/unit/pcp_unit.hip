@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 
 #include "../pcp32.hpp"
+#include "../pcp_pair_schedule.hpp"
 
 using namespace pcp;
 
@@ -18,6 +19,24 @@ void unit_split(long n, const double *u, long nc, int *inside, long *cell, float
 // below_edge of the cells i[k]
 void unit_below_edge(long n, const long *i, double dx, double *x) {
   for (long k = 0; k < n; ++k) x[k] = below_edge(i[k], dx);
+}
+
+// the unlike pairs of a cell of nel electrons and nion ions, chain after chain:
+// particle of the less and of the more numerous species; returns their number,
+// or -1 where a chain past long_chains holds more than one
+long unit_unlike_pairs(int nel, int nion, int *near_, int *far_) {
+  UnlikeChains U;
+  U.set(nel, nion);
+  long n = 0;
+  for (int e = 0; e < U.n; ++e) {
+    const int len = U.length(e);
+    if (len > 1 && e >= U.long_chains() && U.big != U.n) return -1;
+    for (int j = 0; j < len; ++j, ++n) {
+      near_[n] = e;
+      far_[n] = U.partner(e, j);
+    }
+  }
+  return n;
 }
 
 // sort keys of the global cells (cr[k], cz[k]) of a grid of Dr x Dz domains of
