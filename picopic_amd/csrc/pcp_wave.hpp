@@ -125,7 +125,9 @@ __device__ __forceinline__ float run_sum_f(float x, const Runs &R) {
 // particle kernels are bound by instruction issue and spent 15 to 30 % of it
 // on run sums).  A masked infinity would leave NaN in the next run: only for
 // values that run_sums_bounded accepts.  A DPP read needs two instructions
-// between it and the write of its register: the other values' steps.
+// between it and the write of its register: the other values' steps.  The sums
+// are written while masks of later steps are unread, so they share no register
+// with an input (the &).
 #define PCP_RUN_FMA(x, m, ctrl) "v_fmac_f32_dpp %" #x ", %" #x ", %" #m " " ctrl " bank_mask:0xf bound_ctrl:0\n\t"
 #define PCP_RUN_FMA3(m, ctrl) PCP_RUN_FMA(0, m, ctrl) PCP_RUN_FMA(1, m, ctrl) PCP_RUN_FMA(2, m, ctrl)
 #define PCP_RUN_FMA4(m, ctrl) PCP_RUN_FMA3(m, ctrl) PCP_RUN_FMA(3, m, ctrl)
@@ -136,7 +138,7 @@ __device__ __forceinline__ void run_sums_f(float &a, float &b, float &c, const R
                    PCP_RUN_FMA3(5, "row_shr:4 row_mask:0xf") PCP_RUN_FMA3(6, "row_shr:8 row_mask:0xf")
                        PCP_RUN_FMA3(7, "row_bcast:15 row_mask:0xa")
                            PCP_RUN_FMA3(8, "row_bcast:31 row_mask:0xc") "s_nop 1"
-               : "+v"(a), "+v"(b), "+v"(c)
+               : "+&v"(a), "+&v"(b), "+&v"(c)
                : "v"(run_mask_f(R, 0)), "v"(run_mask_f(R, 1)), "v"(run_mask_f(R, 2)), "v"(run_mask_f(R, 3)),
                  "v"(run_mask_f(R, 4)), "v"(run_mask_f(R, 5)));
 }
@@ -146,7 +148,7 @@ __device__ __forceinline__ void run_sums_f(float &a, float &b, float &c, float &
                    PCP_RUN_FMA4(6, "row_shr:4 row_mask:0xf") PCP_RUN_FMA4(7, "row_shr:8 row_mask:0xf")
                        PCP_RUN_FMA4(8, "row_bcast:15 row_mask:0xa")
                            PCP_RUN_FMA4(9, "row_bcast:31 row_mask:0xc") "s_nop 1"
-               : "+v"(a), "+v"(b), "+v"(c), "+v"(d)
+               : "+&v"(a), "+&v"(b), "+&v"(c), "+&v"(d)
                : "v"(run_mask_f(R, 0)), "v"(run_mask_f(R, 1)), "v"(run_mask_f(R, 2)), "v"(run_mask_f(R, 3)),
                  "v"(run_mask_f(R, 4)), "v"(run_mask_f(R, 5)));
 }

@@ -3,12 +3,61 @@
 // this file).
 #include <hip/hip_runtime.h>
 
+#include <initializer_list>
+#include <utility>
+
 #include "../pcp32.hpp"
 #include "../pcp_pair_schedule.hpp"
+#include "../pcp_wave.hpp"
 
 using namespace pcp;
 
+namespace {
+
+// Run sums along the runs of equal keys of a wavefront of x and of masks of the
+// runs themselves (0 or 1).  FORM 4 and 3: four and three values at once (the
+// masks dead after it), 1: value by value.
+template <int FORM>
+__global__ void k_run_sums(const uint32_t *key, const float *x, float *out) {
+  const Runs R = runs_of(key[threadIdx.x]);
+  float a[4] = {run_mask_f(R, 5), run_mask_f(R, 1), run_mask_f(R, 4), x[threadIdx.x]};
+  if (FORM == 4) run_sums_f(a[0], a[1], a[2], a[3], R);
+  if (FORM == 3) run_sums_f(a[0], a[1], a[2], R);
+  for (int k = 0; k < 4; ++k) out[k * 64 + threadIdx.x] = FORM == 1 ? run_sum_f(a[k], R) : a[k];
+}
+
+// a kernel's arrays on the device: inputs copied in, outputs copied back
+template <class F>
+int on_device(std::initializer_list<std::pair<const void *, size_t>> in, void *out, size_t out_bytes, F launch) {
+  void *d[5] = {};
+  int n = 0, rc = 0;
+  for (const auto &a : in) {
+    if (hipMalloc(&d[n], a.second) != hipSuccess ||
+        hipMemcpy(d[n], a.first, a.second, hipMemcpyHostToDevice) != hipSuccess)
+      rc = -1;
+    ++n;
+  }
+  if (hipMalloc(&d[n], out_bytes) != hipSuccess) rc = -1;
+  if (rc == 0) {
+    launch(d, d[n]);
+    if (hipGetLastError() != hipSuccess || hipMemcpy(out, d[n], out_bytes, hipMemcpyDeviceToHost) != hipSuccess) rc = -1;
+  }
+  for (void *p : d) (void)hipFree(p);
+  return rc;
+}
+
+}  // namespace
+
 extern "C" {
+
+int unit_run_sums(int form, const uint32_t *key, const float *x, float *out) {
+  return on_device({{key, 64 * sizeof(uint32_t)}, {x, 64 * sizeof(float)}}, out, 4 * 64 * sizeof(float),
+                   [form](void **d, void *o) {
+                     auto f = form == 4 ? k_run_sums<4> : form == 3 ? k_run_sums<3> : k_run_sums<1>;
+                     hipLaunchKernelGGL(f, dim3(1), dim3(64), 0, 0, (const uint32_t *)d[0], (const float *)d[1],
+                                        (float *)o);
+                   });
+}
 
 // split_coordinate of n coordinates u of a grid of nc cells: inside[k], and
 // where inside the cell and the offset
