@@ -26,6 +26,14 @@ __global__ void k_run_sums(const uint32_t *key, const float *x, float *out) {
   for (int k = 0; k < 4; ++k) out[k * 64 + threadIdx.x] = FORM == 1 ? run_sum_f(a[k], R) : a[k];
 }
 
+// reserve_groups of a wavefront: head, size and rank of every lane
+__global__ void k_reserve_groups(const uint32_t *key, const int *active, int *out) {
+  const ReserveGroup G = reserve_groups(key[threadIdx.x], active[threadIdx.x] != 0);
+  out[threadIdx.x] = G.head;
+  out[64 + threadIdx.x] = (int)G.size;
+  out[128 + threadIdx.x] = (int)G.rank;
+}
+
 // a kernel's arrays on the device: inputs copied in, outputs copied back
 template <class F>
 int on_device(std::initializer_list<std::pair<const void *, size_t>> in, void *out, size_t out_bytes, F launch) {
@@ -56,6 +64,14 @@ int unit_run_sums(int form, const uint32_t *key, const float *x, float *out) {
                      auto f = form == 4 ? k_run_sums<4> : form == 3 ? k_run_sums<3> : k_run_sums<1>;
                      hipLaunchKernelGGL(f, dim3(1), dim3(64), 0, 0, (const uint32_t *)d[0], (const float *)d[1],
                                         (float *)o);
+                   });
+}
+
+int unit_reserve_groups(const uint32_t *key, const int *active, int *out) {
+  return on_device({{key, 64 * sizeof(uint32_t)}, {active, 64 * sizeof(int)}}, out, 3 * 64 * sizeof(int),
+                   [](void **d, void *o) {
+                     hipLaunchKernelGGL(k_reserve_groups, dim3(1), dim3(64), 0, 0, (const uint32_t *)d[0],
+                                        (const int *)d[1], (int *)o);
                    });
 }
 

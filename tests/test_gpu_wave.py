@@ -38,3 +38,41 @@ def test_joined_run_sums_equal_the_single_ones(lengths):
     assert np.abs(one[3] - total)[last].max() <= 64 * 2.0 ** -24 * np.abs(x).sum()
     assert np.array_equal(four[:, last], one[:, last])
     assert np.array_equal(three[:3, last], one[:3, last])
+
+
+def patterns():
+    rng = np.random.default_rng(7)
+    lane = np.arange(64)
+    yield "one", np.zeros(64), np.ones(64)
+    yield "two in turn", lane % 2, np.ones(64)
+    yield "eight in turn", lane % 8, np.ones(64)
+    yield "nine in turn", lane % 9, np.ones(64)
+    yield "all different", lane, np.ones(64)
+    yield "sorted", lane // 7, np.ones(64)
+    yield "eight runs, two keys", lane // 8 % 2, np.ones(64)
+    yield "two in turn, half inactive", lane % 2, lane // 2 % 2
+    yield "none", lane, np.zeros(64)
+    yield "last", lane, lane == 63
+    for n in (3, 12, 40):
+        yield "random %d" % n, rng.integers(0, n, 64), rng.random(64) < 0.8
+
+
+@pytest.mark.parametrize("name,key,active", list(patterns()), ids=[p[0] for p in patterns()])
+def test_reserving_lanes_form_groups(name, key, active):
+    """Every active lane has a place of its own among its key's, and few lanes ask: one a run, and where there are
+    more than eight runs at most one for each of eight keys."""
+    key, active = key.astype(np.uint32) + 5, active.astype(np.int32)
+    out = np.zeros((3, 64), np.int32)
+    print("groups", name, flush=True)
+    assert unit().unit_reserve_groups(ptr(key), ptr(active), ptr(out)) == 0
+    head, size, rank = (a[active != 0] for a in out)
+    k, lanes = key[active != 0], np.flatnonzero(active)
+    for h in np.unique(head):
+        g = head == h
+        assert h in lanes and len(np.unique(k[g])) == 1 and k[g][0] == key[h]
+        assert (size[g] == g.sum()).all() and np.array_equal(np.sort(rank[g]), np.arange(g.sum()))
+    runs = int(active[0] + ((active[1:] != 0) & ((key[1:] != key[:-1]) | (active[:-1] == 0))).sum())
+    asked, different = len(np.unique(head)), len(np.unique(k))
+    assert asked <= runs
+    if runs > 8 and different <= 8:
+        assert asked == different
