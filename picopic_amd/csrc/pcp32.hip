@@ -563,7 +563,7 @@ __global__ void __launch_bounds__(256) k32_push_mom(Geom g, FieldsT<float> f, Sp
       const bool live = key != DEAD_CELL;
       float q[7] = {live ? 1.f : 0.f, w, w * v[0], w * v[1], w * v[2], w * v[2] * v[2],
                     w * (v[0] * v[0] + v[1] * v[1])};
-      if (run_sums_bounded(q)) {
+      if (run_sums_bounded(abs_sum(q))) {
         run_sums_f(q[0], q[1], q[2], q[3], R);
         run_sums_f(q[4], q[5], q[6], R);
       } else {

@@ -156,15 +156,17 @@ __device__ __forceinline__ void run_sums_f(float &a, float &b, float &c, float &
 #undef PCP_RUN_FMA3
 #undef PCP_RUN_FMA4
 
-// every lane's values are numbers, small enough that the sum of 64 of them is
-// finite (a NaN fails the comparison)
+// sum of the magnitudes of a lane's values
 template <int N>
-__device__ __forceinline__ bool run_sums_bounded(const float (&q)[N]) {
+__device__ __forceinline__ float abs_sum(const float (&q)[N]) {
   float s = fabsf(q[0]);
 #pragma unroll
   for (int k = 1; k < N; ++k) s += fabsf(q[k]);
-  return __all(s < 0x1p120f);
+  return s;
 }
+// every lane's values (their abs_sum t) are numbers, small enough that the sum
+// of 64 of them is finite (a NaN fails the comparison)
+__device__ __forceinline__ bool run_sums_bounded(float t) { return __all(t < 0x1p120f); }
 
 // Compensated summation in FP32.  two_sum returns fl(a + b) and sets e to
 // its rounding error, a + b - fl(a + b), exactly (Knuth's branch-free

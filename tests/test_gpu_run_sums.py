@@ -57,3 +57,26 @@ def test_run_sums(ccs, domains, ppc):
     assert hit.any() and np.abs(mixed).max() > 2.0 ** 120
     assert np.abs(got - mixed)[~hit].max() <= 2e-5 * np.abs(light).max()
     assert np.abs(got - mixed)[hit].max() <= 2e-5 * np.abs(mixed).max()
+
+
+@pytest.mark.parametrize("ccs,domains", [("zigzag", (1, 1)), ("zigzag", (2, 2)), ("vb", (2, 2))])
+def test_particles_at_rest_deposit_nothing(ccs, domains):
+    """Wavefronts of particles at rest skip the sums; with one moving particle among them its current is the oracle's."""
+    cell = 1e-6
+    n = 150
+    size = (GRID[0] * cell, GRID[1] * cell)
+    r, z = np.full(n, 3.375 * cell), np.full(n, 5.625 * cell)
+    w, ids = np.full(n, 1e6), np.arange(n, dtype=np.uint64)
+    for moving in (0, 1):
+        v = np.zeros((3, n))
+        v[:, 70] = moving * np.array([3e7, 2e7, -4e7])
+        out = []
+        print("rest", ccs, domains, moving, flush=True)
+        for make in (oracle, device):
+            s, add = make(size, GRID, domains, 0.25 * cell / 3e8, [(-1, 1, False)], ccs, n)
+            add(0, r, z, *v, w, ids)
+            s.step(1)
+            out.append(s.get_grid("J")[:, :, 2:-2, 2:-2])
+        if ccs == "zigzag" and not moving:
+            assert not out[1].any()
+        assert np.abs(out[1] - out[0]).max() <= 2e-5 * np.abs(out[0]).max()
