@@ -316,10 +316,21 @@ struct MapParts32 {
 
 // Order of the particles for the map deposit.  Its run sums need equal cells
 // next to each other: as the sorts leave them, but a species just uploaded may
-// be in any order.  k_map_heads counts the places where the cell changes along
-// the storage; where that is more than every fourth, an index list in cell
-// order is made (count, scan, fill), which the deposit then follows.
-__device__ __forceinline__ bool map_in_order(const uint32_t *heads, long n) { return (long)*heads * 4 <= n; }
+// be in any order.  Where map_may_list allows it, k_map_heads counts the places
+// where the cell changes along the storage; where that is more than every fourth
+// and more than the cells, an index list in cell order is made (count,
+// scan, fill), which the deposit then follows.  (Sorted cells of few particles
+// have many such places, at most one a cell, and nothing to gain.)
+__device__ __forceinline__ bool map_listed(const uint32_t *heads, long n, long ncells) {
+  return heads && (long)*heads * 4 > n && (long)*heads > ncells;
+}
+// The list pays for itself in the atomics of the quantities besides the density
+// that it saves, from about 2^18 values a map on.  Unsorted FP64 particles,
+// without and with it: momentum of 65,536 100 and 105 us, of 131,072 150 and 125,
+// of 4.2 M 3,150 and 1,370; energy of 131,072 95 and 115, of 524,288 245 and 217.
+// The density alone is faster without (131,072: 66 and 106 us, 4.2 M: 865 and
+// 972), and small maps are launches (1,024: 34 and 78 us).
+static bool map_may_list(long n, int qn) { return qn > 0 && n * (1 + qn) > (1L << 18); }
 
 template <class V>
 __global__ void __launch_bounds__(256) k_map_heads(Geom g, V parts, long n, uint32_t *heads) {
@@ -334,8 +345,9 @@ __global__ void __launch_bounds__(256) k_map_heads(Geom g, V parts, long n, uint
 }
 
 template <class V>
-__global__ void __launch_bounds__(256) k_map_count(Geom g, V parts, long n, const uint32_t *heads, uint32_t *cnt) {
-  if (map_in_order(heads, n)) return;
+__global__ void __launch_bounds__(256) k_map_count(Geom g, V parts, long n, long ncells, const uint32_t *heads,
+                                                   uint32_t *cnt) {
+  if (!map_listed(heads, n, ncells)) return;
   for (long b = (long)blockIdx.x * blockDim.x; b < n; b += (long)gridDim.x * blockDim.x) {
     const long p = b + threadIdx.x;
     const uint32_t c = p < n ? parts.cell(g, p) : NO_CELL;
@@ -344,9 +356,9 @@ __global__ void __launch_bounds__(256) k_map_count(Geom g, V parts, long n, cons
 }
 
 template <class V>
-__global__ void __launch_bounds__(256) k_map_fill(Geom g, V parts, long n, const uint32_t *heads, const uint32_t *off,
-                                                  uint32_t *fill, uint32_t *perm) {
-  if (map_in_order(heads, n)) return;
+__global__ void __launch_bounds__(256) k_map_fill(Geom g, V parts, long n, long ncells, const uint32_t *heads,
+                                                  const uint32_t *off, uint32_t *fill, uint32_t *perm) {
+  if (!map_listed(heads, n, ncells)) return;
   for (long b = (long)blockIdx.x * blockDim.x; b < n; b += (long)gridDim.x * blockDim.x) {
     const long p = b + threadIdx.x;
     const uint32_t c = p < n ? parts.cell(g, p) : NO_CELL;
@@ -364,11 +376,11 @@ __global__ void __launch_bounds__(256) k_map_fill(Geom g, V parts, long n, const
 // the deposit, which reads six arrays through it).
 // QN quantities besides the density -- 0: none, 1: momentum_abs_w (energy),
 // 3: momentum_w (temperature, momentum)
-template <class V, int QN>
-__global__ void __launch_bounds__(256) k_map_deposit(Geom g, V parts, long n, double mass, const uint32_t *heads,
-                                                     const uint32_t *n_live, const uint32_t *perm, double *N,
-                                                     double *Q) {
-  const bool listed = !map_in_order(heads, n);
+template <int QN, class V>
+__global__ void __launch_bounds__(256) k_map_deposit(Geom g, V parts, long n, double mass, long ncells,
+                                                     const uint32_t *heads, const uint32_t *n_live,
+                                                     const uint32_t *perm, double *N, double *Q) {
+  const bool listed = map_listed(heads, n, ncells);
   const long m = listed ? (long)*n_live : n;
   const long DP = (long)g.Dr * g.Dz * g.P;
   for (long b = (long)blockIdx.x * blockDim.x; b < m; b += (long)gridDim.x * blockDim.x) {
@@ -480,38 +492,40 @@ __global__ void k_zero_f64(double *p, long n) {
 
 }  // namespace
 
-// the deposit of map `kind` (the sort's key, counters and scan storage, free
-// between sorts, hold the index list in cell order where one is needed)
-template <class V>
-static int map_deposit(pcp_ctx *c, V parts, long n, double mass, int kind, double *N, double *PW, double *PABS) {
+// the deposit of QN quantities besides the density (the sort's key, counters and
+// scan storage, free between sorts, hold the index list in cell order where one
+// is needed)
+template <int QN, class V>
+static int map_deposit(pcp_ctx *c, V parts, long n, double mass, double *N, double *Q) {
   const Geom &g = c->g;
   const long ncells = (long)c->D * g.nr * g.nz;
-  const unsigned gz = (unsigned)std::min<long>((ncells + 256) / 256, (long)c->n_cu * 16);
   const unsigned gp = (unsigned)std::max(1L, std::min((n + 255) / 256, (long)c->n_cu * 16));
   // the last of the fill counters (one more than the cells) counts the order's breaks
-  uint32_t *heads = c->sort_fill + ncells;
-  hipLaunchKernelGGL(k_zero_u32, dim3(gz), dim3(256), 0, c->stream, c->sort_count, c->sort_fill, ncells + 1);
-  // few workgroups: each ends with an atomic on the one counter
-  const unsigned gh = std::min(gp, (unsigned)c->n_cu * 4);
-  hipLaunchKernelGGL(k_map_heads<V>, dim3(gh), dim3(256), 0, c->stream, g, parts, n, heads);
-  hipLaunchKernelGGL(k_map_count<V>, dim3(gp), dim3(256), 0, c->stream, g, parts, n, heads, c->sort_count);
-  size_t bytes = c->sort_temp_bytes;
-  if (hipcub::DeviceScan::ExclusiveSum(c->sort_temp, bytes, c->sort_count, c->sort_offset, (int)(ncells + 1),
-                                       c->stream) != hipSuccess)
-    return -1;
-  hipLaunchKernelGGL(k_map_fill<V>, dim3(gp), dim3(256), 0, c->stream, g, parts, n, heads, c->sort_offset,
-                     c->sort_fill, c->sort_key);
-  const uint32_t *n_live = c->sort_offset + ncells;
-  if (kind == 0)
-    hipLaunchKernelGGL((k_map_deposit<V, 0>), dim3(gp), dim3(256), 0, c->stream, g, parts, n, mass, heads, n_live,
-                       c->sort_key, N, N);
-  else if (kind == 2)
-    hipLaunchKernelGGL((k_map_deposit<V, 1>), dim3(gp), dim3(256), 0, c->stream, g, parts, n, mass, heads, n_live,
-                       c->sort_key, N, PABS);
-  else
-    hipLaunchKernelGGL((k_map_deposit<V, 3>), dim3(gp), dim3(256), 0, c->stream, g, parts, n, mass, heads, n_live,
-                       c->sort_key, N, PW);
+  uint32_t *heads = map_may_list(n, QN) ? c->sort_fill + ncells : nullptr;
+  if (heads) {
+    const unsigned gz = (unsigned)std::min<long>((ncells + 256) / 256, (long)c->n_cu * 16);
+    hipLaunchKernelGGL(k_zero_u32, dim3(gz), dim3(256), 0, c->stream, c->sort_count, c->sort_fill, ncells + 1);
+    // few workgroups: each ends with an atomic on the one counter
+    const unsigned gh = std::min(gp, (unsigned)c->n_cu * 4);
+    hipLaunchKernelGGL(k_map_heads<V>, dim3(gh), dim3(256), 0, c->stream, g, parts, n, heads);
+    hipLaunchKernelGGL(k_map_count<V>, dim3(gp), dim3(256), 0, c->stream, g, parts, n, ncells, heads, c->sort_count);
+    size_t bytes = c->sort_temp_bytes;
+    if (hipcub::DeviceScan::ExclusiveSum(c->sort_temp, bytes, c->sort_count, c->sort_offset, (int)(ncells + 1),
+                                         c->stream) != hipSuccess)
+      return -1;
+    hipLaunchKernelGGL(k_map_fill<V>, dim3(gp), dim3(256), 0, c->stream, g, parts, n, ncells, heads, c->sort_offset,
+                       c->sort_fill, c->sort_key);
+  }
+  hipLaunchKernelGGL((k_map_deposit<QN, V>), dim3(gp), dim3(256), 0, c->stream, g, parts, n, mass, ncells, heads,
+                     c->sort_offset + ncells, c->sort_key, N, Q);
   return 0;
+}
+// the deposit of map `kind`
+template <class V>
+static int map_deposit_kind(pcp_ctx *c, V parts, long n, double mass, int kind, double *N, double *PW, double *PABS) {
+  if (kind == 0) return map_deposit<0>(c, parts, n, mass, N, N);
+  if (kind == 2) return map_deposit<1>(c, parts, n, mass, N, PABS);
+  return map_deposit<3>(c, parts, n, mass, N, PW);
 }
 
 int launch_species_map(pcp_ctx *c, int sp, int kind, double *N, double *PW, double *PABS, double *OUT) {
@@ -526,10 +540,10 @@ int launch_species_map(pcp_ctx *c, int sp, int kind, double *N, double *PW, doub
   int rc = 0;
   if (c->s32) {
     Species32 &s = c->s32->sp[sp];
-    if (s.n > 0) rc = map_deposit(c, MapParts32{s, c->cur, g.Nz, g.dr, g.dz}, s.n, mass, kind, N, PW, PABS);
+    if (s.n > 0) rc = map_deposit_kind(c, MapParts32{s, c->cur, g.Nz, g.dr, g.dz}, s.n, mass, kind, N, PW, PABS);
   } else {
     SpeciesDev &s = c->sp[sp];
-    if (s.n > 0) rc = map_deposit(c, MapParts64{s, c->cur}, s.n, mass, kind, N, PW, PABS);
+    if (s.n > 0) rc = map_deposit_kind(c, MapParts64{s, c->cur}, s.n, mass, kind, N, PW, PABS);
   }
   if (rc < 0) return rc;
   const long cells = (long)c->D * g.nr * g.nz;
