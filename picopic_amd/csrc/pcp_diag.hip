@@ -283,7 +283,8 @@ struct MapParts64 {
   // its global cell r_cell Nz + z_cell; NO_CELL when removed or outside the grid
   __device__ __forceinline__ uint32_t cell(const Geom &g, long p) const {
     const double r = s.r[cur][p], z = s.z[cur][p];
-    if (!(r >= 0)) return NO_CELL;
+    // (after the phase "move" the coordinates may be anything)
+    if (!(r >= 0) || !isfinite(r) || !isfinite(z)) return NO_CELL;
     const int cr = cell_number(r, g.dr), cz = cell_number(z, g.dz);
     return cr < g.Nr && cz >= 0 && cz < g.Nz ? (uint32_t)cr * (uint32_t)g.Nz + (uint32_t)cz : NO_CELL;
   }

@@ -57,3 +57,21 @@ def test_maps_do_not_depend_on_the_storage_order(precision, n, order):
         assert np.abs(first[k] - again).max() <= 1e-12 * scale, k
         # FP32: positions rounded to 2^-24 of a cell against clouds that reach a node with 1e-3 of a cell or more
         assert np.abs(first[k] - ref[k]).max() <= (1e-12 if precision == "fp64" else 1e-4) * scale, k
+
+
+@pytest.mark.parametrize("vz", [np.inf, -np.inf, 1e300, 4e8])
+def test_particles_outside_the_grid_are_in_no_map(vz):
+    """Between the phases "move" and "migrate" a particle may lie anywhere, also at an infinite longitude."""
+    size, grid = (8e-3, 8e-3), (8, 8)
+    maps = []
+    for n in (2, 3):
+        ctx = capi.Context(size, grid, (2, 2), 1e-10, [(-1, 1, True, 16)])
+        x, zero = np.full(n, 4.2e-3), np.zeros(n)
+        v = np.array([1e6, 2e6, vz])[:n]
+        ctx.upload(0, x, x, zero, zero, v, zero + 1e6)
+        print("outside", n, vz, flush=True)
+        ctx.phase("move")
+        maps.append([ctx.species_map(0, k)[:, :, 2:-2, 2:-2] for k in ("density", "energy", "momentum")])
+    for a, b in zip(*maps):
+        assert np.isfinite(a).all() and a.any()
+        assert np.abs(a - b).max() <= 1e-12 * np.abs(a).max()
