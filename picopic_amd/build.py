@@ -32,7 +32,9 @@ FLAGS = [
 # The FP32 split kernels carry FP64 only where FP32 is not enough (the VB
 # terms, the deposit end point); there one-ulp reciprocal-based division and
 # approximate library functions suffice (6 % faster on the VB workload), so
-# that file alone is built with them.  The FP64 kernels keep IEEE division.
+# that file alone is built with them.  The FP64 kernels' quotients round as IEEE
+# division does; those of ordinary operands leave out its scaling and special
+# cases (quot and recip).
 # The collision pairs' FP64 constants are rebuilt from literals where they are
 # used instead of being kept in registers over the pair loop (180 instead of
 # 250 registers; 6.7 -> 5.4 ms per pass at the third wavefront per SIMD); the

@@ -1022,7 +1022,7 @@ __global__ void k32_init_bunch(Geom g, Species32 s, long base, long n_new, doubl
     s.vphi[0][q] = s.vphi[1][q] = 0.f;
     s.vz[0][q] = s.vz[1][q] = (float)vz;
     s.w[q] = (float)weight;
-    int d = (int)((long)floor(r / g.dr) / g.nr) * g.Dz + (int)((long)floor(z / g.dz) / g.nz);
+    const int d = domain_of(g, cell_number(r, g.dr), cell_number(z, g.dz));
     s.seq[q] = gbase[(long)d * MAX_SPECIES + sp] + (uint64_t)p;
     s.id[q] = (uint64_t)q;
   }

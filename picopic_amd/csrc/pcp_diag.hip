@@ -58,7 +58,7 @@ struct Pos32 {
 // add sign * q of the ring cloud at (r, z) to the control volumes
 __device__ void add_cloud(double *Q, long ldq, double r, double z, double dr, double dz, double q) {
   const double vc = PI * ((r + dr / 2) * (r + dr / 2) - (r - dr / 2) * (r - dr / 2)) * dz;
-  const int i0 = (int)floor(r / dr), k0 = (int)floor(z / dz);
+  const int i0 = cell_number(r, dr), k0 = cell_number(z, dz);
   for (int i = i0; i <= i0 + 1; ++i) {
     const double a0 = fmax(0.0, (i - 0.5) * dr), a1 = (i + 0.5) * dr;
     const double lo = fmax(a0, r - dr / 2), hi = fmin(a1, r + dr / 2);

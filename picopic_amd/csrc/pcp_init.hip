@@ -76,7 +76,7 @@ __global__ void k_init_bunch(Geom g, SpeciesDev s, long base, long n_new, double
     s.vphi[q] = 0;
     s.vz[q] = vz;
     s.w[q] = weight;
-    int d = (int)((long)floor(r / g.dr) / g.nr) * g.Dz + (int)((long)floor(z / g.dz) / g.nz);
+    const int d = domain_of(g, cell_number(r, g.dr), cell_number(z, g.dz));
     s.seq[q] = gbase[(long)d * MAX_SPECIES + sp] + (uint64_t)p;
     s.id[q] = (uint64_t)q;
   }

@@ -343,10 +343,10 @@ __global__ void k_migrate(Geom g, SpeciesDev s, int sp, int cur, StepState *st, 
     double r = s.r[cur][p], z = s.z[cur][p];
     double ro = s.r[cur ^ 1][p], zo = s.z[cur ^ 1][p];
     if (r < 0 || ro < 0) { s.r[cur][p] = -1; continue; }
-    long cr = bad_position(r, z) ? -1 : (long)floor(r / g.dr);
-    long cz = bad_position(r, z) ? -1 : (long)floor(z / g.dz);
+    const int cr = bad_position(r, z) ? -1 : cell_number(r, g.dr);
+    const int cz = bad_position(r, z) ? -1 : cell_number(z, g.dz);
     if (cr < 0 || cz < 0 || cr >= g.Nr || cz >= g.Nz) { s.r[cur][p] = -1; continue; }
-    int d_new = domain_of(g, (int)cr, (int)cz);
+    int d_new = domain_of(g, cr, cz);
     int d_old = domain_of(g, cell_number(ro, g.dr), cell_number(zo, g.dz));
     if (d_new != d_old) append_migrant(mg, st, sp, p, d_old, d_new, s.seq[p], g, &err);
   }

@@ -9,6 +9,7 @@
 #include <hip/hip_runtime.h>
 #include <hipcub/hipcub.hpp>
 
+#include "pcp_physics.hpp"
 #include "pcp_sort.hpp"
 #include "pcp_wave.hpp"
 
@@ -24,7 +25,7 @@ __global__ void __launch_bounds__(SORT_BLOCK) k_sort_count(Geom g, SpeciesDev s,
       uint32_t k = sentinel;
       const double r = s.r[cur][p], z = s.z[cur][p];
       if (r >= 0) {
-        const long cr = (long)floor(r / g.dr), cz = (long)floor(z / g.dz);
+        const int cr = cell_number(r, g.dr), cz = cell_number(z, g.dz);
         const int I = (int)g.div_nr.div((uint32_t)cr), J = (int)g.div_nz.div((uint32_t)cz);
         const int d = I * g.Dz + J;
         k = sort_cell_key(g, d, cr - (long)I * g.nr, cz - (long)J * g.nz);

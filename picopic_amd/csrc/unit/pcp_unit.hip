@@ -8,6 +8,7 @@
 
 #include "../pcp32.hpp"
 #include "../pcp_pair_schedule.hpp"
+#include "../pcp_physics.hpp"
 #include "../pcp_wave.hpp"
 
 using namespace pcp;
@@ -32,6 +33,18 @@ __global__ void k_reserve_groups(const uint32_t *key, const int *active, int *ou
   out[threadIdx.x] = G.head;
   out[64 + threadIdx.x] = (int)G.size;
   out[128 + threadIdx.x] = (int)G.rank;
+}
+
+// out[0] a / b, out[1] a / b with b's reciprocal at hand, out[2] sqrt(b),
+// out[3] a / c^2, out[4] the cell of a in cells of size b
+__global__ void k_quotients(long n, const double *a, const double *b, double *out) {
+  for (long k = (long)blockIdx.x * blockDim.x + threadIdx.x; k < n; k += (long)gridDim.x * blockDim.x) {
+    out[k] = quot(a[k], b[k]);
+    out[n + k] = quot(a[k], b[k], recip(b[k]));
+    out[2 * n + k] = sqrt_normal(b[k]);
+    out[3 * n + k] = over_c2(a[k]);
+    out[4 * n + k] = (double)cell_number(a[k], b[k]);
+  }
 }
 
 // a kernel's arrays on the device: inputs copied in, outputs copied back
@@ -72,6 +85,14 @@ int unit_reserve_groups(const uint32_t *key, const int *active, int *out) {
                    [](void **d, void *o) {
                      hipLaunchKernelGGL(k_reserve_groups, dim3(1), dim3(64), 0, 0, (const uint32_t *)d[0],
                                         (const int *)d[1], (int *)o);
+                   });
+}
+
+int unit_quotients(long n, const double *a, const double *b, double *out) {
+  return on_device({{a, n * sizeof(double)}, {b, n * sizeof(double)}}, out, 5 * n * sizeof(double),
+                   [n](void **d, void *o) {
+                     hipLaunchKernelGGL(k_quotients, dim3(1024), dim3(256), 0, 0, n, (const double *)d[0],
+                                        (const double *)d[1], (double *)o);
                    });
 }
 
