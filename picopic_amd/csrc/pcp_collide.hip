@@ -53,7 +53,7 @@ struct View64 {
     if (!(r >= 0)) return false;
     cr = cell_number(r, g.dr);
     cz = cell_number(s.z[cur][p], g.dz);
-    return true;
+    return cr < g.Nr && cz >= 0 && cz < g.Nz;   // (the phase "move" may leave the grid)
   }
   __device__ __forceinline__ void load(long p, double v[3]) const {
     v[0] = s.vr[p]; v[1] = s.vphi[p]; v[2] = s.vz[p];

@@ -4,7 +4,7 @@
 // (the gather becomes broadcast loads) and their current nodes (the
 // wave-aggregated atomics issue one add per node).  The counting and
 // scatter passes aggregate their counters per workgroup chunk in LDS.  Removed particles
-// (r < 0) are dropped; the tail [n_live, n) is marked removed so that the
+// (r < 0) and those outside the grid are dropped; the tail [n_live, n) is marked removed so that the
 // host-side slot count stays valid without a synchronisation.
 #include <hip/hip_runtime.h>
 #include <hipcub/hipcub.hpp>
@@ -24,8 +24,9 @@ __global__ void __launch_bounds__(SORT_BLOCK) k_sort_count(Geom g, SpeciesDev s,
     table_count_chunk(t, c0, s.n, sentinel, count, [&](long p) {
       uint32_t k = sentinel;
       const double r = s.r[cur][p], z = s.z[cur][p];
-      if (r >= 0) {
-        const int cr = cell_number(r, g.dr), cz = cell_number(z, g.dz);
+      const int cr = cell_number(r, g.dr), cz = cell_number(z, g.dz);
+      // (after the phase "move" a particle may lie past the grid)
+      if (r >= 0 && cr < g.Nr && cz >= 0 && cz < g.Nz) {
         const int I = (int)g.div_nr.div((uint32_t)cr), J = (int)g.div_nz.div((uint32_t)cz);
         const int d = I * g.Dz + J;
         k = sort_cell_key(g, d, cr - (long)I * g.nr, cz - (long)J * g.nz);

@@ -67,3 +67,23 @@ def test_sort_orders_by_cell_and_keeps_every_particle(precision, domains, case):
     dom = (cr // nr_d) * domains[1] + cz // nz_d
     key = dom * 10 ** 12 + cr * 10 ** 6 + cz
     assert np.all(np.diff(key) >= 0)
+
+
+def test_particles_past_the_grid_are_dropped():
+    """Between the phases "move" and "migrate" a beam's particles may lie past the grid: the sort drops them, as the
+    collector would, and a collision pass leaves them out."""
+    from picopic_amd import capi
+    size, grid, n = (8e-3, 8e-3), (8, 8), 40
+    rng = np.random.default_rng(9)
+    ctx = capi.Context(size, grid, (2, 2), 1e-10, [(-1, 1, True, 64), (1, 1836, False, 64)])
+    r, z, zero = rng.uniform(1e-3, 6e-3, n), rng.uniform(1e-3, 5e-3, n), np.zeros(n)
+    vr, vz = np.zeros(n), np.full(n, 1e6)
+    vz[::4], vr[1::4], vz[2::4] = 2e8, 2e8, -2e8
+    ctx.upload(0, r, z, vr, zero, vz, zero + 1e6)
+    ctx.upload(1, r, z, zero, zero, zero, zero + 1e6)
+    print("past the grid", flush=True)
+    ctx.phase("move")
+    ctx.collide("ta77s", 0, 1, 1, 0)
+    ctx.sort(0)
+    inside = (r + vr * 1e-10 < size[0]) & (z + vz * 1e-10 < size[1]) & (z + vz * 1e-10 >= 0)
+    assert 0 < inside.sum() < n and ctx.count(0) == inside.sum()
