@@ -290,6 +290,12 @@ __device__ __forceinline__ void push_one(const Geom &g, const Fields &f, double 
 __device__ __forceinline__ bool bad_position(double r, double z) {
   return isnan(r) || isinf(r) || isnan(z) || isinf(z);
 }
+// position outside the grid, where the phase "move" may leave a particle until
+// "migrate" collects it: it has neither fields nor current there
+__device__ __forceinline__ bool outside_grid(const Geom &g, double r, double z) {
+  const int cr = cell_number(r, g.dr), cz = cell_number(z, g.dz);
+  return bad_position(r, z) || cr < 0 || cz < 0 || cr >= g.Nr || cz >= g.Nz;
+}
 
 __global__ void __launch_bounds__(256) k_push(Geom g, Fields f, SpeciesDev s, int cur, StepState *st) {
   int err = 0;
@@ -297,6 +303,7 @@ __global__ void __launch_bounds__(256) k_push(Geom g, Fields f, SpeciesDev s, in
     double r = s.r[cur][p], z = s.z[cur][p];
     if (r < 0) continue;
     if (bad_position(r, z)) { err |= ERR_NAN_POSITION; continue; }
+    if (outside_grid(g, r, z)) continue;
     double v[3] = {s.vr[p], s.vphi[p], s.vz[p]};
     push_one(g, f, s.q, s.m, r, z, v, &err);
     s.vr[p] = v[0]; s.vphi[p] = v[1]; s.vz[p] = v[2];
@@ -483,7 +490,7 @@ __global__ void k_mark(Geom g, SpeciesDev s, int sp, int cur, StepState *st, uin
   for (long p = (long)blockIdx.x * blockDim.x + threadIdx.x; p < s.n; p += (long)gridDim.x * blockDim.x) {
     double r = s.r[cur][p], z = s.z[cur][p];
     double ro = s.r[cur ^ 1][p], zo = s.z[cur ^ 1][p];
-    if (r < 0 || ro < 0) continue;
+    if (r < 0 || ro < 0 || outside_grid(g, r, z)) continue;
     if (!vb_is_strict_reset(g.dr, g.dz, r, z, ro, zo)) continue;
     int d = domain_of(g, cell_number(r, g.dr), cell_number(z, g.dz));
     Dom dm = make_dom(g, d);
@@ -503,7 +510,7 @@ __global__ void __launch_bounds__(256) k_deposit_exact(Geom g, Fields f, Species
   for (long p = (long)blockIdx.x * blockDim.x + threadIdx.x; p < s.n; p += (long)gridDim.x * blockDim.x) {
     double r = s.r[cur][p], z = s.z[cur][p];
     double ro = s.r[cur ^ 1][p], zo = s.z[cur ^ 1][p];
-    if (r < 0 || ro < 0) continue;
+    if (r < 0 || ro < 0 || outside_grid(g, r, z)) continue;
     int d = domain_of(g, cell_number(r, g.dr), cell_number(z, g.dz));
     Dom dm = make_dom(g, d);
     double w = s.w[p];

@@ -91,3 +91,34 @@ def test_faster_than_light_is_an_error(precision, pusher, speed):
         with pytest.raises(capi.PcpError, match="0x2|0x3"):
             ctx.step(1)
             ctx.sync()
+
+
+@pytest.mark.parametrize("ccs", ["zigzag", "vb"])
+def test_phases_before_the_collector_leave_out_particles_past_the_grid(ccs):
+    """Deposit and push between the phases "move" and "migrate": particles past the walls have no cell; the others'
+    current and velocities are those of a run without them."""
+    from picopic_amd import capi
+    size, grid, dt = (8e-3, 8e-3), (8, 8), 2e-12
+    rng = np.random.default_rng(4)
+    n, m = 40, 10
+    r, z = rng.uniform(1e-3, 6e-3, n + m), rng.uniform(1e-3, 6e-3, n + m)
+    vr, vz, zero = rng.normal(0, 1e7, n + m), rng.normal(0, 1e7, n + m), np.zeros(n + m)
+    r[n:n + m // 2], vr[n:n + m // 2] = 7.9e-3, 2e8
+    z[n + m // 2:], vz[n + m // 2:] = 7.9e-3, 2e8
+    out = []
+    print("before the collector", ccs, flush=True)
+    for k in (n, n + m):
+        ctx = capi.Context(size, grid, (2, 2), dt, [(-1, 1, True, 64)], ccs=ccs)
+        ctx.upload(0, r[:k], z[:k], vr[:k], zero[:k], vz[:k], zero[:k] + 1e6, np.arange(k, dtype=np.uint64))
+        E, H, Hat = Hh.random_fields(np.random.default_rng(5), 4, 4, 4)
+        for name, a in (("E", E), ("H", H), ("H_at_et", Hat)):
+            ctx.set_grid(name, a)
+        for ph in ("move", "deposit", "push", "migrate"):
+            ctx.phase(ph)
+        p = _by_id(ctx.particles(0))
+        out.append((ctx.get_grid("J"), p))
+        assert len(p["id"]) == n
+    (ja, a), (jb, b) = out
+    assert np.abs(ja).max() > 0 and np.abs(ja - jb).max() <= 1e-12 * np.abs(ja).max()
+    for k in ("r", "z", "vr", "vz"):
+        assert np.array_equal(a[k], b[k]), k
