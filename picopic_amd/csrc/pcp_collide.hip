@@ -123,7 +123,7 @@ __global__ void __launch_bounds__(256) k_coll_count(Geom g, V v, uint32_t *cnt, 
     const long p = b0 + threadIdx.x;
     const uint32_t k = bucket_of(g, v, p, n, sentinel, mask);
     const bool a = k != sentinel;
-    (void)run_reserve(cnt, k, a);
+    (void)group_reserve(cnt, k, a);
   }
 }
 
@@ -141,7 +141,7 @@ __global__ void __launch_bounds__(256) k_coll_fill(Geom g, V v, const uint32_t *
     const long p = b0 + threadIdx.x;
     const uint32_t k = bucket_of(g, v, p, n, sentinel, mask);
     const bool a = k != sentinel;
-    const uint32_t slot = run_reserve(fill, k, a);
+    const uint32_t slot = group_reserve(fill, k, a);
     if (a) perm[off[k] + slot] = (uint32_t)p;
   }
 }

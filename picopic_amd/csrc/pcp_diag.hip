@@ -352,7 +352,7 @@ __global__ void __launch_bounds__(256) k_map_count(Geom g, V parts, long n, long
   for (long b = (long)blockIdx.x * blockDim.x; b < n; b += (long)gridDim.x * blockDim.x) {
     const long p = b + threadIdx.x;
     const uint32_t c = p < n ? parts.cell(g, p) : NO_CELL;
-    (void)run_reserve(cnt, c, c != NO_CELL);
+    (void)group_reserve(cnt, c, c != NO_CELL);
   }
 }
 
@@ -363,7 +363,7 @@ __global__ void __launch_bounds__(256) k_map_fill(Geom g, V parts, long n, long 
   for (long b = (long)blockIdx.x * blockDim.x; b < n; b += (long)gridDim.x * blockDim.x) {
     const long p = b + threadIdx.x;
     const uint32_t c = p < n ? parts.cell(g, p) : NO_CELL;
-    const uint32_t slot = run_reserve(fill, c, c != NO_CELL);
+    const uint32_t slot = group_reserve(fill, c, c != NO_CELL);
     if (c != NO_CELL) perm[off[c] + slot] = (uint32_t)p;
   }
 }
