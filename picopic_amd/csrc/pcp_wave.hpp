@@ -257,6 +257,7 @@ __device__ __forceinline__ RunLinks run_links(uint32_t key, const Runs &R) {
 // past it.  All 64 lanes must call it.
 struct RunSpan {
   int head, next;
+  unsigned long long heads;   // the first lanes of all runs
 };
 __device__ __forceinline__ RunSpan run_span(uint32_t key) {
   const int lane = __lane_id();
@@ -264,7 +265,7 @@ __device__ __forceinline__ RunSpan run_span(uint32_t key) {
   const unsigned long long heads = __ballot(lane == 0 || prev != key);
   const unsigned long long after = lane == 63 ? 0ull : heads & (~0ull << (lane + 1));
   return RunSpan{63 - __clzll((long long)(heads & (~0ull >> (63 - lane)))),
-                 after ? __ffsll((long long)after) - 1 : 64};
+                 after ? __ffsll((long long)after) - 1 : 64, heads};
 }
 
 // The lanes that reserve together: `head` asks for `size` slots, of which the
@@ -288,7 +289,7 @@ __device__ __forceinline__ ReserveGroup reserve_groups(uint32_t key, bool active
   const RunSpan r = run_span(k);
   ReserveGroup G{r.head, (uint32_t)(r.next - r.head), (uint32_t)(lane - r.head)};
   unsigned long long left = __ballot(active);
-  if (__popcll(left & __ballot(lane == r.head)) > MERGE_RUNS) {
+  if (__popcll(left & r.heads) > MERGE_RUNS) {
     for (int t = 0; t < MERGE_RUNS && left; ++t) {
       const int first = __ffsll((long long)left) - 1;
       const unsigned long long m = __ballot(k == (uint32_t)__builtin_amdgcn_readlane((int)k, first));
@@ -303,6 +304,7 @@ __device__ __forceinline__ ReserveGroup reserve_groups(uint32_t key, bool active
 // slots of the active lanes' keys counted up in ctr, one atomic a group; all 64
 // lanes call it
 __device__ __forceinline__ uint32_t group_reserve(uint32_t *ctr, uint32_t key, bool active) {
+  if (!__any(active)) return 0;   // most wavefronts of a list of few cells
   const ReserveGroup G = reserve_groups(key, active);
   uint32_t base = 0;
   if (active && (int)__lane_id() == G.head) base = atomicAdd(ctr + key, G.size);
