@@ -12,18 +12,20 @@
 //                   32, 64, 128, 256 or more particles of either species; a
 //                   cell missing a species ends its r-row as the reference's
 //                   `break` does)
-//   k_coll_prep     per group of listed cells (1024 particle slots of one
-//                   size class, one workgroup; a cell above 256 has a
-//                   workgroup and a global stage of its own):
-//                   shuffle each bucket by ranking its particles on
-//                   a Philox key of (particle id, pass), per-cell sums in the
-//                   shuffled order, density / temperature / Debye length, and
-//                   the first cell of each r-row whose values are not normal
-//                   (the reference's `break` ends the rest of that row)
-//   k_coll_pairs    per group, the same way: the reference's pair schedule as
+//   k_coll_prep     per group of listed cells (512 particle slots of one size
+//                   class, one workgroup): shuffle each bucket by ranking its
+//                   particles on a Philox key of (particle id, pass), and the
+//                   per-cell sums in the shuffled order
+//   k_coll_stats    per listed cell, a lane each: density / temperature / Debye
+//                   length, and the first cell of each r-row whose values are
+//                   not normal (the reference's `break` ends the rest of that
+//                   row)
+//   k_coll_pairs    per group (1024 slots): the reference's pair schedule as
 //                   dense lists of independent pairs over the group's cells,
 //                   velocities staged in FP64; pair q of global cell c draws
 //                   the uniforms Philox(seed; c << 24 | q, 2 pass + 1)
+// A cell above 256 has a workgroup and a global stage of its own
+// (k_coll_prep_crowd, with its statistics, and k_coll_pairs_crowd).
 #include <hip/hip_runtime.h>
 #include <hipcub/hipcub.hpp>
 
@@ -372,8 +374,8 @@ struct GroupEntries {
 // place, are ranked again by (key, id, index)).  The sums run in the shuffled
 // order, one thread per (quantity, species, cell).  Bound by latency: the
 // bitonic sort and one-thread sums of a wavefront per cell took 6.2 ms per pass
-// on a million cells of 32 + 32 FP64 particles on average (16 wavefronts per CU
-// at a 1024-slot stage still 2.7), this 2.1 with k_coll_stats.
+// on a million cells of 32 + 32 FP64 particles on average (the ranks at a
+// 1024-slot stage, 12 wavefronts per CU, still 2.7), this 2.1 with k_coll_stats.
 template <class V>
 __global__ void __launch_bounds__(COLL_GROUP_BLOCK) k_coll_prep(Geom g, V ve, V vi, const uint32_t *off_e,
                                                                 const uint32_t *off_i, uint32_t *perm_e,
