@@ -73,3 +73,33 @@ def test_beam_as_wide_as_the_grid(precision, domains, radius):
     for s in (orc, dev):
         s.step(2)
     assert orc.count(1) == dev.count(1)
+
+
+@pytest.mark.parametrize("beam", [False, True])
+@pytest.mark.parametrize("grid,domains", [((2, 2), (1, 1)), ((8, 16), (2, 2)), ((9, 7), (3, 1))])
+@pytest.mark.parametrize("ccs", ["zigzag", "vb"])
+def test_moves_next_to_the_walls_stay_in_the_grid(ccs, grid, domains, beam):
+    """FP32 steps of particles within 2^-26 .. 2^-2 of a cell of walls and corners, at all speeds: every stored cell is
+    one of the grid's, before and after a sort, and the maps of the particles are finite."""
+    n = 4000
+    rng = np.random.default_rng(grid[0] + 10 * beam)
+    dt = 0.5 * CELL / 3e8
+    edge = 2.0 ** -rng.uniform(2, 26, (2, n))
+    # plasma is mirrored half a cell inside the walls, a beam only at the axis
+    low, high = (0.5, 0.5) if not beam else (0.5, 0.0)
+    u = np.where(rng.random(n) < 0.5, low + edge[0], grid[0] - high - edge[0])
+    w = np.where(rng.random(n) < 0.5, (0.0 if beam else 0.5) + edge[1], grid[1] - high - edge[1])
+    v = rng.normal(size=(3, n))
+    v *= 10.0 ** rng.uniform(-6, 8.4, n) / np.linalg.norm(v, axis=0)
+    ctx = capi.Context((grid[0] * CELL, grid[1] * CELL), grid, domains, dt, [(-1, 1, beam, n)], ccs=ccs,
+                       precision="fp32")
+    ctx.upload(0, u * CELL, w * CELL, *v, np.full(n, 1e3))
+    print("walls", ccs, grid, domains, beam, flush=True)
+    for _ in range(3):
+        ctx.step(1)
+        p = check(ctx, grid)
+        assert len(p["r"]) and (p["r"] >= 0).all() and (p["z"] >= 0).all()
+        assert beam or len(p["r"]) == n
+        ctx.sort(0)
+        assert ctx.count(0) == len(p["r"])
+        assert all(np.isfinite(ctx.species_map(0, k)).all() for k in ("density", "momentum"))
